@@ -40,7 +40,8 @@ EXACT_FLAGS = {"quantize.hip": ["-ffp-contract=off"], "generic.hip": ["-ffp-cont
 # (v_accvgpr_read) sits between each MFMA and its scaling. No kernel in
 # these files needs scratch memory with it.
 VGPR_MFMA = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
-UNIT_FLAGS = {**EXACT_FLAGS, **{f: VGPR_MFMA for f in ("gemv_mfma.hip", "vrow_b2.hip", "vrow_b4.hip", "vrow_b8.hip")}}
+UNIT_FLAGS = {**EXACT_FLAGS, **{f: VGPR_MFMA for f in ("gemv_mfma.hip", "vrow_b2.hip", "vrow_b4.hip", "vrow_b8.hip",
+                                                     "xgemm_b2.hip", "xgemm_b4.hip", "xgemm_b8.hip")}}
 
 
 def _sources() -> list[pathlib.Path]:

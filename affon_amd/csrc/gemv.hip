@@ -1,4 +1,6 @@
-// rocm_quantized_matmul.gemv — HBM-bound decode kernel for small M.
+// rocm_quantized_matmul.gemv — HBM-bound decode kernel for small M. Batches
+// go to the matrix-core kernels of xgemm.h wherever those take the problem
+// and are ahead (see gemv_launch).
 //
 // Counterpart of the reference's SIMD decode paths (metal simd1/simd4,
 // docs/core/quantized-inference.md:136-149): fused unpack, affine decode and
@@ -312,6 +314,18 @@ hipError_t gemv_group_launch(const QmmProblem* group, int count, const Launch& l
   }
 }
 
+namespace {
+// Up to four rows cost this file's kernel one pass over the weights. Where
+// its decode is cheap (8-bit codes; 2-bit codes a word at a time) and the
+// matrix-core kernel would have to split K to fill the GPU, which costs a
+// second launch, the one pass is ahead: 2 x 4096 x 4096 f32 at 8 bits 12.0
+// against 15.5 us, 2-bit groups of 32 2 x 4096 x 4160 11.8 against 16.1; from
+// 128 column tiles on it is behind (14336 columns: 30.2 against 20.9).
+bool one_pass_is_ahead(const QmmProblem& p) {
+  return p.M <= 4 && p.N <= 8192 && (p.bits == 8 || (p.bits == 2 && p.group % 64 != 0));
+}
+}  // namespace
+
 hipError_t gemv_launch(const QmmProblem& p, const Launch& l) {
   hipStream_t stream = l.stream;
   if (p.epi.kind == kEpiSiluPair && !gemv_pair_supports(p)) return hipErrorInvalidValue;
@@ -322,6 +336,7 @@ hipError_t gemv_launch(const QmmProblem& p, const Launch& l) {
       default: return gemv1_launch_b8(p, stream);
     }
   }
+  if (!one_pass_is_ahead(p) && xgemm_supports(p)) return xgemm_launch(p, l);
   switch (p.bits) {
     case 2: return launch_bits<2>(p, stream);
     case 4: return launch_bits<4>(p, stream);

@@ -97,6 +97,11 @@ constexpr int kMaxGroup = 4;
 bool gemv_group_supports(const QmmProblem* group, int count);
 hipError_t gemv_group_launch(const QmmProblem* group, int count, const Launch& l);
 
+// The general matrix-core kernels (xgemm.h) that gemv_launch runs where the
+// M = 1 kernel does not take the problem.
+bool xgemm_supports(const QmmProblem& p);
+hipError_t xgemm_launch(const QmmProblem& p, const Launch& l);
+
 bool gemv_mfma_supports(const QmmProblem& p);
 hipError_t gemv_mfma_launch(const QmmProblem& p, const Launch& l);
 // Grouped launch of 2..4 problems on the LDS-tiled kernel (decode batches

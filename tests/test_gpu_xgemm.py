@@ -1,0 +1,145 @@
+"""GPU: the general matrix-core kernels (f32 activations split into three bf16
+planes, any group that is a multiple of 32, any K of whole groups) at the edges
+of their tiles, K units and parameter windows."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import affon_amd as A
+from affon_amd import _native
+from tests.helpers import HipRuntime, pack_codes, storage, widened
+
+pytestmark = pytest.mark.gpu
+
+# Rows around the kernels' tiles of 16, 32, 64 and 128; columns around their 64, 128 and 256.
+SHAPES = [(2, 65), (5, 1), (16, 64), (17, 63), (32, 130), (33, 127), (64, 129), (65, 300), (129, 257)]
+# (K, group): half a step at the end, one unit and less, odd blocks per group,
+# more groups than one parameter window, K ranges over workgroups.
+DEPTHS = [(64, 32), (160, 32), (96, 96), (576, 192), (1376, 32), (1344, 64), (2560, 128), (4160, 64)]
+
+
+def operands(rng, M, N, K, bits, group, x_dtype, p_dtype):
+    q = rng.integers(0, 1 << bits, size=(N, K))
+    x = storage(rng.standard_normal((M, K)), x_dtype)
+    s = storage(rng.uniform(0.5, 1.5, (N, K // group)) / (1 << bits), p_dtype)
+    b = storage(rng.standard_normal((N, K // group)), p_dtype)
+    return x, q, s, b
+
+
+def upload_all(session, x, q, s, b, bits, x_dtype, p_dtype):
+    return (session.from_bytes(x, A.TensorSpec(x_dtype, x.shape)),
+            session.from_bytes(pack_codes(q, bits), A.TensorSpec("u32", (q.shape[0], q.shape[1] * bits // 32))),
+            session.from_bytes(s, A.TensorSpec(p_dtype, s.shape)), session.from_bytes(b, A.TensorSpec(p_dtype, b.shape)))
+
+
+def expected_and_bound(x, q, s, b, group):
+    """The product in f64, and what f32 sums of its terms may be off by: a
+    term is rounded in its product with s or b and once per addition above
+    it, at most one per 16 values of k in its K part, the planes' three
+    chains and the parts' reduction."""
+    x, s, b = (widened(v).astype(np.float64) for v in (x, s, b))
+    s, b = np.repeat(s, group, 1), np.repeat(b, group, 1)
+    depth = x.shape[1] / 16 + 32
+    return x @ (s * q + b).T, depth * 2.0 ** -24 * (np.abs(x) @ (s * q + np.abs(b)).T)
+
+
+@pytest.mark.parametrize("x_dtype,p_dtype", [("f32", "f32"), ("f32", "bf16"), ("bf16", "bf16"), ("bf16", "f32")])
+@pytest.mark.parametrize("bits", [2, 4, 8])
+def test_edges_against_f64(session, bits, x_dtype, p_dtype, rng):
+    for i, (K, group) in enumerate(DEPTHS):
+        for M, N in SHAPES[i % 2::2] if K > 600 else SHAPES:
+            if K * bits % 128:
+                continue
+            x, q, s, b = operands(rng, M, N, K, bits, group, x_dtype, p_dtype)
+            t = upload_all(session, x, q, s, b, bits, x_dtype, p_dtype)
+            out = session.tensor(np.full((M, N), np.nan, np.float32))
+            A.quantized_matmul_into(out, *t, bits=bits, group_size=group, implementation="gemv")
+            want, bound = expected_and_bound(x, q, s, b, group)
+            err = np.abs(out.numpy() - want)
+            assert (err <= bound).all(), (M, N, K, group, float((err / bound).max()))
+            # Far below the bound in norm: no plane, block or part is missing.
+            assert np.linalg.norm(err) <= 2e-6 * np.linalg.norm(want), (M, N, K, group)
+
+
+@pytest.mark.parametrize("M", [3, 40, 200])
+def test_extreme_activations(session, M):
+    """One nonzero activation per row: the largest finite f32 (no plane
+    overflows), one with all 24 bits set, a small normal one, infinities and a
+    NaN; codes 1 with scale 2^-10 and bias 0 give x * 2^-10 exactly."""
+    N, K, group = 70, 320, 64
+    values = np.array([np.finfo(np.float32).max, np.float32(1.0 + 2.0 ** -23), -np.float32(2.0 ** -100 * (2 - 2.0 ** -23)),
+                       np.inf, -np.inf, np.nan], np.float32)
+    x = np.zeros((M, K), np.float32)
+    picked = values[np.arange(M) % len(values)]
+    x[np.arange(M), np.arange(M) * 7 % K] = picked
+    q, s, b = np.ones((N, K), np.int64), np.full((N, K // group), 2.0 ** -10, np.float32), np.zeros((N, K // group), np.float32)
+    t = upload_all(session, x, q, s, b, 4, "f32", "f32")
+    out = session.empty("f32", (M, N))
+    A.quantized_matmul_into(out, *t, bits=4, group_size=group, implementation="gemv")
+    # The bias term 0 * sum(x) makes an infinite row NaN, as on the VALU kernel.
+    want = np.where(np.isfinite(picked), picked * np.float32(2.0 ** -10), np.nan).astype(np.float32)
+    np.testing.assert_array_equal(out.numpy(), np.broadcast_to(want[:, None], (M, N)))
+    # With a positive bias an infinite row stays infinite.
+    t = t[:3] + (session.tensor(np.full_like(b, 0.25)),)
+    A.quantized_matmul_into(out, *t, bits=4, group_size=group, implementation="gemv")
+    rows = np.isinf(picked)
+    np.testing.assert_array_equal(out.numpy()[rows], np.broadcast_to(picked[rows, None], (rows.sum(), N)))
+
+
+@pytest.mark.parametrize("M", [6, 24, 100, 300])
+def test_epilogues_and_repeats(session, M, rng):
+    """Output bias and SiLU-gated product through the K ranges' reduction and
+    without it; repeated runs are bit-identical."""
+    for N, K in ((200, 4096), (96, 192)):
+        x, q, s, b = operands(rng, M, N, K, 4, 64, "f32", "f32")
+        t = upload_all(session, x, q, s, b, 4, "f32", "f32")
+        y = A.quantized_matmul(*t, bits=4, group_size=64).numpy()
+        np.testing.assert_array_equal(A.quantized_matmul(*t, bits=4, group_size=64).numpy(), y)
+        bias = rng.standard_normal(N).astype(np.float32)
+        fused = A.quantized_linear(*t, session.tensor(bias), bits=4, group_size=64).numpy()
+        np.testing.assert_array_equal(fused, y + bias)
+        _, q2, s2, b2 = operands(rng, M, N, K, 4, 64, "f32", "f32")
+        up = upload_all(session, x, q2, s2, b2, 4, "f32", "f32")
+        u = A.quantized_matmul(*up, bits=4, group_size=64).numpy().astype(np.float64)
+        g = y.astype(np.float64)
+        want = g / (1 + np.exp(-g)) * u
+        got = A.quantized_silu_gate(t[0], t[1:], up[1:], bits=4, group_size=64).numpy()
+        # expf, the division and the product: a few roundings of the result.
+        assert (np.abs(got - want) <= 8 * 2.0 ** -24 * np.abs(want) + 1e-30).all()
+
+
+@pytest.mark.parametrize("M", [8, 128])
+def test_capture_without_scratch(M, rng):
+    """Captured on a session whose workspace is still empty, the product runs
+    in one K range; replays give the same bits each time, within the bound."""
+    from affon_amd import ops
+    N, K, group = 256, 4160, 64
+    x, q, s, b = operands(rng, M, N, K, 8, group, "f32", "bf16")
+    hip = HipRuntime()
+    with A.Session("rocm") as session:
+        t = upload_all(session, x, q, s, b, 8, "f32", "bf16")
+        out = session.empty("f32", (M, N))
+        desc = ops._descriptor(*t, 8, group, out, "auto", "backend_equivalent")
+        lib = _native.load()
+
+        def enqueue():
+            assert lib.affon_rocm_quantized_matmul(session._handle, ctypes.byref(desc)) == 0, _native.last_error()
+
+        graph = hip.capture(session.stream, enqueue)
+        try:
+            want, bound = expected_and_bound(x, q, s, b, group)
+            first = None
+            for _ in range(3):
+                zeros = np.zeros((M, N), np.float32)
+                _native.check(lib.affon_rocm_memcpy_h2d(session._handle, out.data_ptr, zeros.ctypes.data, zeros.nbytes),
+                              "clear")
+                hip.replay(session.stream, graph)
+                session.synchronize()
+                got = out.numpy()
+                assert (np.abs(got - want) <= bound).all()
+                first = got if first is None else first
+                np.testing.assert_array_equal(got, first)
+                A.quantized_matmul(*t, bits=8, group_size=group)
+        finally:
+            hip.destroy(graph)
