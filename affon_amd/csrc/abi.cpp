@@ -910,7 +910,10 @@ int affon_rocm_softmax(affon_rocm_session* session, const void* x, int32_t dtype
   int status = check_rows(x, dtype, rows, cols, out, "softmax");
   if (status != AFFON_ROCM_OK) return status;
   if ((status = check_session(session)) != AFFON_ROCM_OK) return status;
-  hipError_t e = affon::softmax_launch(x, dtype, rows, cols, out, session->stream);
+  affon::Launch launch;
+  launch.stream = session->stream;
+  launch.workspace = session->workspace;
+  hipError_t e = affon::softmax_launch(x, dtype, rows, cols, out, launch);
   if (e != hipSuccess) return hip_fail(e, "softmax");
   return AFFON_ROCM_OK;
 }

@@ -142,7 +142,7 @@ hipError_t quantize_launch(const void* weights, int weight_dtype, int64_t rows, 
                            int param_dtype, hipStream_t stream);
 hipError_t rms_norm_launch(const void* x, int dtype, int64_t rows, int64_t cols, float epsilon, void* out,
                            hipStream_t stream);
-hipError_t softmax_launch(const void* x, int dtype, int64_t rows, int64_t cols, void* out, hipStream_t stream);
+hipError_t softmax_launch(const void* x, int dtype, int64_t rows, int64_t cols, void* out, const Launch& l);
 hipError_t index_select_launch(const void* x, int dtype, int64_t rows, int64_t cols, int axis, const int64_t* index,
                                int64_t count, void* out, hipStream_t stream);
 // One launch that reads every whole 16-byte chunk of up to four buffers once

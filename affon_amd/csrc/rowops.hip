@@ -6,12 +6,19 @@
 // rms_norm(x)[r, c] = x[r, c] / sqrt(mean_c(x[r, :]^2) + epsilon) and
 // softmax(x)[r, c] = exp(x[r, c] - max_r) / sum_c exp(x[r, c] - max_r), both
 // computed in f32 (bf16 inputs widened exactly, bf16 outputs rounded to
-// nearest even), one wave per row. index_select copies whole rows (axis 0)
-// or gathers columns (axis 1); an index outside [0, size) selects zeros
-// (the reference's and PyTorch's behaviour,
-// test/parity/reference/probe-capabilities.py:150-153). All of them are
-// HBM-bound; rows are read once.
+// nearest even). index_select copies whole rows (axis 0) or gathers columns
+// (axis 1); an index outside [0, size) selects zeros (the reference's and
+// PyTorch's behaviour, test/parity/reference/probe-capabilities.py:150-153).
+// All of them are HBM-bound, and latency-bound where the rows are few; a
+// softmax of few long rows by its exponentials. Each row takes as many
+// threads as give each about four 16-byte loads in flight, against one wave
+// per row with one element per lane and load before. Device us, before ->
+// now: softmax f32 32 x 128256 1307 -> 17, 512 x 128256 2482 -> 152 (3.4 TB/s),
+// 512 x 4096 43 -> 13; rms_norm f32 32 x 4096 19.5 -> 4.1, bf16 512 x 4096
+// 23.3 -> 6.0. The sums of many short partial sums are also nearer: softmax
+// over 128256 values 3.3e-6 -> 7.5e-8 off 64 bits.
 
+#include <algorithm>
 #include <type_traits>
 
 #include "device.h"
@@ -20,120 +27,349 @@
 namespace affon {
 namespace {
 
-constexpr int kRowThreads = 256;  // four rows per workgroup, one per wave
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef u32x4_t u32x4_word_t __attribute__((aligned(4)));  // 16 bytes at an f32
+typedef u32x4_t u32x4_half_t __attribute__((aligned(2)));  // 16 bytes at a bf16
 
+// 16 bytes of a row: rows start at any element, the memory takes vectors there.
 template <typename T>
-__device__ __forceinline__ float load_value(const uint8_t* base, int64_t i) {
-  return T::load(base, i);
-}
+struct Vec {
+  static constexpr int kValues = 16 / T::bytes;
+  using unaligned_t = typename std::conditional<T::bytes == 2, u32x4_half_t, u32x4_word_t>::type;
+  float v[kValues];
+  // Values i*kValues .. of a row of cols; those past its end are `fill`.
+  __device__ __forceinline__ void load(const uint8_t* row, int64_t i, int64_t cols, float fill) {
+    const int64_t at = i * kValues;
+    if (at + kValues <= cols) {
+      const u32x4_t raw = *reinterpret_cast<const unaligned_t*>(row + at * T::bytes);
+#pragma unroll
+      for (int e = 0; e < kValues; ++e) {
+        if constexpr (T::bytes == 2)
+          v[e] = __uint_as_float(e % 2 ? raw[e / 2] & 0xffff0000u : raw[e / 2] << 16);
+        else
+          v[e] = __uint_as_float(raw[e]);
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < kValues; ++e) v[e] = at + e < cols ? T::load(row, at + e) : fill;
+    }
+  }
+  __device__ __forceinline__ void store(uint8_t* row, int64_t i, int64_t cols) const {
+    const int64_t at = i * kValues;
+    if (at + kValues <= cols) {
+      u32x4_t raw;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if constexpr (T::bytes == 2)
+          raw[e] = f32_to_bf16_bits(v[2 * e]) | static_cast<uint32_t>(f32_to_bf16_bits(v[2 * e + 1])) << 16;
+        else
+          raw[e] = __float_as_uint(v[e]);
+      }
+      *reinterpret_cast<unaligned_t*>(row + at * T::bytes) = raw;
+    } else {
+#pragma unroll
+      for (int e = 0; e < kValues; ++e)
+        if (at + e < cols) {
+          if constexpr (T::bytes == 2)
+            reinterpret_cast<uint16_t*>(row)[at + e] = f32_to_bf16_bits(v[e]);
+          else
+            reinterpret_cast<float*>(row)[at + e] = v[e];
+        }
+    }
+  }
+};
 
-template <typename T>
-__device__ __forceinline__ void store_value(uint8_t* base, int64_t i, float v) {
-  if constexpr (T::bytes == 2) {
-    reinterpret_cast<uint16_t*>(base)[i] = f32_to_bf16_bits(v);
-  } else {
-    reinterpret_cast<float*>(base)[i] = v;
+constexpr int kAhead = 4;  // vectors a thread has in flight
+
+// f(index, vector) over a thread's vectors of a row, kAhead loads at a time.
+template <typename T, typename F>
+__device__ __forceinline__ void for_vectors(const uint8_t* row, int64_t cols, int64_t first, int64_t end, int step,
+                                            float fill, F&& f) {
+  for (int64_t i = first; i < end; i += static_cast<int64_t>(kAhead) * step) {
+    Vec<T> vec[kAhead];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j)
+      if (i + j * step < end) vec[j].load(row, i + j * step, cols, fill);
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j)
+      if (i + j * step < end) f(i + j * step, vec[j]);
   }
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
+// Combines one value per thread of the THREADS that hold a row (64: a wave;
+// more: the workgroup), the same result in every thread.
+template <int THREADS, typename V, typename F>
+__device__ __forceinline__ V row_reduce(V v, F&& combine) {
 #pragma unroll
-  for (int offset = 32; offset > 0; offset >>= 1) v += __shfl_xor(v, offset);
-  return v;
-}
-
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int offset = 32; offset > 0; offset >>= 1) v = fmaxf(v, __shfl_xor(v, offset));
-  return v;
-}
-
-template <typename T>
-__global__ __launch_bounds__(kRowThreads) void rms_norm_kernel(const uint8_t* x, uint8_t* out, int64_t rows,
-                                                               int64_t cols, float epsilon) {
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * (kRowThreads / 64) + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (row >= rows) return;
-  const int64_t base = row * cols;
-  float ss = 0.0f;
-  for (int64_t c = lane; c < cols; c += 64) {
-    const float v = load_value<T>(x, base + c);
-    ss = fmaf(v, v, ss);
+  for (int offset = 32; offset > 0; offset >>= 1) v = combine(v, v.from(offset));
+  if constexpr (THREADS > 64) {
+    __shared__ V part[THREADS / 64];
+    __syncthreads();  // an earlier row's values are read
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = part[0];
+    for (int i = 1; i < THREADS / 64; ++i) v = combine(v, part[i]);
   }
-  ss = wave_sum(ss);
-  const float denominator = sqrtf(ss / static_cast<float>(cols) + epsilon);
-  for (int64_t c = lane; c < cols; c += 64) store_value<T>(out, base + c, load_value<T>(x, base + c) / denominator);
+  return v;
+}
+
+struct Sum {
+  float s;
+  __device__ __forceinline__ Sum from(int offset) const { return Sum{__shfl_xor(s, offset)}; }
+};
+__device__ __forceinline__ Sum add(Sum a, Sum b) { return Sum{a.s + b.s}; }
+
+// The largest value m seen, NaNs skipped (-inf: none), and sum of exp(x - m).
+struct Peak {
+  float m, s;
+  __device__ __forceinline__ Peak from(int offset) const { return Peak{__shfl_xor(m, offset), __shfl_xor(s, offset)}; }
+};
+// exp(x - m) where m may be -inf, the peak of nothing or of -inf alone: 0.
+__device__ __forceinline__ float exp_below(float x, float m) { return expf(x - (m == -INFINITY ? 0.0f : m)); }
+__device__ __forceinline__ Peak add(Peak a, Peak b) {
+  const float m = fmaxf(a.m, b.m);
+  return Peak{m, a.s * exp_below(a.m, m) + b.s * exp_below(b.m, m)};
+}
+// The peak of vectors first, first + step, .. below end.
+template <typename T>
+__device__ __forceinline__ Peak peak_of(const uint8_t* row, int64_t cols, int64_t first, int64_t end, int step) {
+  Peak p{-INFINITY, 0.0f};
+  for_vectors<T>(row, cols, first, end, step, -INFINITY, [&](int64_t, const Vec<T>& x) {
+    float m = p.m;
+#pragma unroll
+    for (int e = 0; e < Vec<T>::kValues; ++e) m = fmaxf(m, x.v[e]);
+    if (m != p.m) p.s *= exp_below(p.m, m);
+    p.m = m;
+#pragma unroll
+    for (int e = 0; e < Vec<T>::kValues; ++e) p.s += exp_below(x.v[e], m);
+  });
+  return p;
+}
+// Writes exp(x - p.m) / p.s. The quotient q = e * (1/s) takes one correction
+// by its exact remainder, which rounds it as the division does: s lies in
+// [1, cols] and e in [0, 1], so nothing overflows, or both are NaN.
+template <typename T>
+__device__ __forceinline__ void write_softmax(const uint8_t* row, uint8_t* out, int64_t cols, int64_t first,
+                                              int64_t end, int step, Peak p) {
+  const float inv = 1.0f / p.s;
+  for_vectors<T>(row, cols, first, end, step, -INFINITY, [&](int64_t i, Vec<T>& x) {
+#pragma unroll
+    for (int e = 0; e < Vec<T>::kValues; ++e) {
+      const float v = expf(x.v[e] - p.m), q = v * inv;
+      x.v[e] = fmaf(fmaf(-p.s, q, v), inv, q);
+    }
+    x.store(out, i, cols);
+  });
+}
+
+// f(row) for this workgroup's rows with THREADS threads to a row: rows of a
+// wave each four to a workgroup, else one row at a time; workgroups stride
+// over what is left (all of a workgroup's threads together where they share
+// a row).
+constexpr int64_t kMaxGrid = int64_t(1) << 20;
+template <int THREADS, typename F>
+__device__ __forceinline__ void for_rows(int64_t rows, F&& f) {
+  constexpr int kPer = THREADS < 256 ? 256 / THREADS : 1;
+  for (int64_t row = static_cast<int64_t>(blockIdx.x) * kPer + (kPer > 1 ? threadIdx.x / THREADS : 0); row < rows;
+       row += static_cast<int64_t>(gridDim.x) * kPer)
+    f(row);
+}
+
+// A row is read twice, the second time from the caches.
+template <typename T, int THREADS>
+__global__ __launch_bounds__(THREADS < 256 ? 256 : THREADS) void rms_norm_kernel(const uint8_t* x, uint8_t* out,
+                                                                                 int64_t rows, int64_t cols,
+                                                                                 float epsilon) {
+  const int t = threadIdx.x % THREADS;
+  const int64_t n = (cols + Vec<T>::kValues - 1) / Vec<T>::kValues;
+  for_rows<THREADS>(rows, [&](int64_t row) {
+    const uint8_t* in = x + row * cols * T::bytes;
+    Sum ss{0.0f};
+    for_vectors<T>(in, cols, t, n, THREADS, 0.0f, [&](int64_t, const Vec<T>& v) {
+#pragma unroll
+      for (int e = 0; e < Vec<T>::kValues; ++e) ss.s = fmaf(v.v[e], v.v[e], ss.s);
+    });
+    ss = row_reduce<THREADS>(ss, [](Sum a, Sum b) { return add(a, b); });
+    const float denominator = sqrtf(ss.s / static_cast<float>(cols) + epsilon);
+    uint8_t* to = out + row * cols * T::bytes;
+    for_vectors<T>(in, cols, t, n, THREADS, 0.0f, [&](int64_t i, Vec<T>& v) {
+#pragma unroll
+      for (int e = 0; e < Vec<T>::kValues; ++e) v.v[e] = v.v[e] / denominator;
+      v.store(to, i, cols);
+    });
+  });
+}
+
+template <typename T, int THREADS>
+__global__ __launch_bounds__(THREADS < 256 ? 256 : THREADS) void softmax_kernel(const uint8_t* x, uint8_t* out,
+                                                                                int64_t rows, int64_t cols) {
+  const int t = threadIdx.x % THREADS;
+  const int64_t n = (cols + Vec<T>::kValues - 1) / Vec<T>::kValues;
+  for_rows<THREADS>(rows, [&](int64_t row) {
+    const uint8_t* in = x + row * cols * T::bytes;
+    const Peak p = row_reduce<THREADS>(peak_of<T>(in, cols, t, n, THREADS), [](Peak a, Peak b) { return add(a, b); });
+    write_softmax<T>(in, out + row * cols * T::bytes, cols, t, n, THREADS, p);
+  });
+}
+
+// Few long rows: each is cut into parts of kPartVectors, a workgroup each,
+// so that the exponentials (about 20 instructions per value, twice; on 32 CUs
+// alone some 20 us of issue for 32 x 128256) spread over the GPU. The first launch leaves every part's peak in `parts`
+// [rows][count], the second combines a row's and writes.
+constexpr int kPartVectors = 1024;
+
+template <typename T>
+__global__ __launch_bounds__(256) void softmax_parts_kernel(const uint8_t* x, int64_t cols, int count, Peak* parts) {
+  const int64_t row = blockIdx.x / count, part = blockIdx.x % count;
+  const int64_t n = (cols + Vec<T>::kValues - 1) / Vec<T>::kValues;
+  const int64_t first = part * kPartVectors, end = min(n, first + kPartVectors);
+  const Peak p = row_reduce<256>(peak_of<T>(x + row * cols * T::bytes, cols, first + threadIdx.x, end, 256),
+                                 [](Peak a, Peak b) { return add(a, b); });
+  if (threadIdx.x == 0) parts[blockIdx.x] = p;
 }
 
 template <typename T>
-__global__ __launch_bounds__(kRowThreads) void softmax_kernel(const uint8_t* x, uint8_t* out, int64_t rows,
-                                                              int64_t cols) {
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * (kRowThreads / 64) + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (row >= rows) return;
-  const int64_t base = row * cols;
-  float peak = -INFINITY;
-  for (int64_t c = lane; c < cols; c += 64) peak = fmaxf(peak, load_value<T>(x, base + c));
-  peak = wave_max(peak);
-  float sum = 0.0f;
-  for (int64_t c = lane; c < cols; c += 64) sum += expf(load_value<T>(x, base + c) - peak);
-  sum = wave_sum(sum);
-  for (int64_t c = lane; c < cols; c += 64) store_value<T>(out, base + c, expf(load_value<T>(x, base + c) - peak) / sum);
+__global__ __launch_bounds__(256) void softmax_write_kernel(const uint8_t* x, uint8_t* out, int64_t cols, int count,
+                                                            const Peak* parts) {
+  const int64_t row = blockIdx.x / count, part = blockIdx.x % count;
+  Peak p{-INFINITY, 0.0f};
+  for (int i = threadIdx.x; i < count; i += 256) p = add(p, parts[row * count + i]);
+  p = row_reduce<256>(p, [](Peak a, Peak b) { return add(a, b); });
+  const int64_t n = (cols + Vec<T>::kValues - 1) / Vec<T>::kValues;
+  const int64_t first = part * kPartVectors, end = min(n, first + kPartVectors);
+  write_softmax<T>(x + row * cols * T::bytes, out + row * cols * T::bytes, cols, first + threadIdx.x, end, 256, p);
 }
 
-// out[i, c] = x[index[i], c] (axis 0) or out[r, i] = x[r, index[i]] (axis 1),
-// one thread per output element; raw element copies (no arithmetic).
+// out[i, :] = x[index[i], :]: raw copies of U-sized pieces, `pieces` to a row,
+// workgroups of 256 pieces of one row (grid y strides over the rows).
+template <typename U>
+__global__ __launch_bounds__(256) void select_rows_kernel(const U* x, U* out, int64_t rows, int64_t pieces,
+                                                          const int64_t* index, int64_t count) {
+  const int64_t p = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (p >= pieces) return;
+  for (int64_t i = blockIdx.y; i < count; i += gridDim.y) {
+    const int64_t sel = index[i];
+    U v{};
+    if (sel >= 0 && sel < rows) v = x[sel * pieces + p];
+    out[i * pieces + p] = v;
+  }
+}
+
+// out[r, i] = x[r, index[i]], one thread per output element.
 template <int BYTES>
-__global__ __launch_bounds__(256) void index_select_kernel(const uint8_t* x, uint8_t* out, int64_t rows, int64_t cols,
-                                                           int axis, const int64_t* index, int64_t count) {
-  const int64_t out_cols = axis == 0 ? cols : count;
-  const int64_t total = (axis == 0 ? count : rows) * out_cols;
+__global__ __launch_bounds__(256) void select_columns_kernel(const uint8_t* x, uint8_t* out, int64_t rows, int64_t cols,
+                                                             const int64_t* index, int64_t count) {
   const int64_t o = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (o >= total) return;
-  const int64_t r = o / out_cols, c = o - r * out_cols;
-  const int64_t sel = index[axis == 0 ? r : c];
-  const int64_t size = axis == 0 ? rows : cols;
+  if (o >= rows * count) return;
+  const int64_t r = o / count, sel = index[o - r * count];
   using U = typename std::conditional<BYTES == 2, uint16_t, uint32_t>::type;
   U v = 0;
-  if (sel >= 0 && sel < size) v = reinterpret_cast<const U*>(x)[axis == 0 ? sel * cols + c : r * cols + sel];
+  if (sel >= 0 && sel < cols) v = reinterpret_cast<const U*>(x)[r * cols + sel];
   reinterpret_cast<U*>(out)[o] = v;
+}
+
+}  // namespace
+
+namespace {
+
+// f(threads) with the threads that share a row of n vectors as a constant:
+// about four vectors each, so that their loads are in flight together.
+template <typename F>
+void with_row_threads(int64_t n, F&& f) {
+  if (n <= 64 * kAhead)
+    f(std::integral_constant<int, 64>{});
+  else if (n <= 512 * kAhead)
+    f(std::integral_constant<int, 256>{});
+  else
+    f(std::integral_constant<int, 1024>{});
+}
+
+template <typename T>
+hipError_t rms_norm_typed(const uint8_t* x, int64_t rows, int64_t cols, float epsilon, uint8_t* out,
+                          hipStream_t stream) {
+  with_row_threads((cols + Vec<T>::kValues - 1) / Vec<T>::kValues, [&](auto threads) {
+    constexpr int kThreads = decltype(threads)::value, kPer = kThreads < 256 ? 256 / kThreads : 1;
+    hipLaunchKernelGGL((rms_norm_kernel<T, kThreads>), dim3(static_cast<unsigned>(std::min(kMaxGrid, (rows + kPer - 1) / kPer))),
+                       dim3(kThreads < 256 ? 256 : kThreads), 0, stream, x, out, rows, cols, epsilon);
+  });
+  return hipGetLastError();
+}
+
+// Rows below which a long row is cut into parts: from about half the CUs on,
+// a workgroup per row fills the GPU and the second launch costs more than it
+// gives.
+constexpr int64_t kFewRows = 128;
+
+template <typename T>
+hipError_t softmax_typed(const uint8_t* x, int64_t rows, int64_t cols, uint8_t* out, const Launch& l) {
+  const int64_t n = (cols + Vec<T>::kValues - 1) / Vec<T>::kValues;
+  const int64_t count = (n + kPartVectors - 1) / kPartVectors;
+  if (rows < kFewRows && count > 1 && count <= (int64_t(1) << 16)) {
+    // Without scratch (a captured stream whose workspace cannot grow): one workgroup per row.
+    if (auto* parts = static_cast<Peak*>(l.scratch(static_cast<size_t>(rows * count) * sizeof(Peak)))) {
+      const dim3 grid(static_cast<unsigned>(rows * count));
+      hipLaunchKernelGGL(softmax_parts_kernel<T>, grid, dim3(256), 0, l.stream, x, cols, static_cast<int>(count), parts);
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return e;
+      hipLaunchKernelGGL(softmax_write_kernel<T>, grid, dim3(256), 0, l.stream, x, out, cols, static_cast<int>(count),
+                         parts);
+      return hipGetLastError();
+    }
+  }
+  with_row_threads(n, [&](auto threads) {
+    constexpr int kThreads = decltype(threads)::value, kPer = kThreads < 256 ? 256 / kThreads : 1;
+    hipLaunchKernelGGL((softmax_kernel<T, kThreads>), dim3(static_cast<unsigned>(std::min(kMaxGrid, (rows + kPer - 1) / kPer))),
+                       dim3(kThreads < 256 ? 256 : kThreads), 0, l.stream, x, out, rows, cols);
+  });
+  return hipGetLastError();
 }
 
 }  // namespace
 
 hipError_t rms_norm_launch(const void* x, int dtype, int64_t rows, int64_t cols, float epsilon, void* out,
                            hipStream_t stream) {
-  const dim3 grid(static_cast<unsigned>((rows + 3) / 4));
   const auto* xi = static_cast<const uint8_t*>(x);
   auto* o = static_cast<uint8_t*>(out);
-  if (dtype == AFFON_ROCM_BF16)
-    hipLaunchKernelGGL(rms_norm_kernel<BF16>, grid, dim3(kRowThreads), 0, stream, xi, o, rows, cols, epsilon);
-  else
-    hipLaunchKernelGGL(rms_norm_kernel<F32>, grid, dim3(kRowThreads), 0, stream, xi, o, rows, cols, epsilon);
-  return hipGetLastError();
+  return dtype == AFFON_ROCM_BF16 ? rms_norm_typed<BF16>(xi, rows, cols, epsilon, o, stream)
+                                  : rms_norm_typed<F32>(xi, rows, cols, epsilon, o, stream);
 }
 
-hipError_t softmax_launch(const void* x, int dtype, int64_t rows, int64_t cols, void* out, hipStream_t stream) {
-  const dim3 grid(static_cast<unsigned>((rows + 3) / 4));
+hipError_t softmax_launch(const void* x, int dtype, int64_t rows, int64_t cols, void* out, const Launch& l) {
   const auto* xi = static_cast<const uint8_t*>(x);
   auto* o = static_cast<uint8_t*>(out);
-  if (dtype == AFFON_ROCM_BF16)
-    hipLaunchKernelGGL(softmax_kernel<BF16>, grid, dim3(kRowThreads), 0, stream, xi, o, rows, cols);
-  else
-    hipLaunchKernelGGL(softmax_kernel<F32>, grid, dim3(kRowThreads), 0, stream, xi, o, rows, cols);
+  return dtype == AFFON_ROCM_BF16 ? softmax_typed<BF16>(xi, rows, cols, o, l) : softmax_typed<F32>(xi, rows, cols, o, l);
+}
+
+namespace {
+template <typename U>
+hipError_t select_rows(const void* x, int64_t rows, int64_t row_bytes, const int64_t* index, int64_t count, void* out,
+                       hipStream_t stream) {
+  const int64_t pieces = row_bytes / static_cast<int64_t>(sizeof(U));
+  const dim3 grid(static_cast<unsigned>((pieces + 255) / 256), static_cast<unsigned>(std::min<int64_t>(count, 32768)));
+  hipLaunchKernelGGL(select_rows_kernel<U>, grid, dim3(256), 0, stream, static_cast<const U*>(x), static_cast<U*>(out),
+                     rows, pieces, index, count);
   return hipGetLastError();
 }
+}  // namespace
 
 hipError_t index_select_launch(const void* x, int dtype, int64_t rows, int64_t cols, int axis, const int64_t* index,
                                int64_t count, void* out, hipStream_t stream) {
-  const int64_t total = (axis == 0 ? count : rows) * (axis == 0 ? cols : count);
-  const dim3 grid(static_cast<unsigned>((total + 255) / 256));
+  const bool half = dtype == AFFON_ROCM_BF16;
+  if (axis == 0) {
+    // Rows in 16-byte pieces where every row starts at one, else by element.
+    const int64_t row_bytes = cols * (half ? 2 : 4);
+    if (row_bytes % 16 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0)
+      return select_rows<u32x4_t>(x, rows, row_bytes, index, count, out, stream);
+    return half ? select_rows<uint16_t>(x, rows, row_bytes, index, count, out, stream)
+                : select_rows<uint32_t>(x, rows, row_bytes, index, count, out, stream);
+  }
+  const dim3 grid(static_cast<unsigned>((rows * count + 255) / 256));
   const auto* xi = static_cast<const uint8_t*>(x);
   auto* o = static_cast<uint8_t*>(out);
-  if (dtype == AFFON_ROCM_BF16)
-    hipLaunchKernelGGL(index_select_kernel<2>, grid, dim3(256), 0, stream, xi, o, rows, cols, axis, index, count);
+  if (half)
+    hipLaunchKernelGGL(select_columns_kernel<2>, grid, dim3(256), 0, stream, xi, o, rows, cols, index, count);
   else
-    hipLaunchKernelGGL(index_select_kernel<4>, grid, dim3(256), 0, stream, xi, o, rows, cols, axis, index, count);
+    hipLaunchKernelGGL(select_columns_kernel<4>, grid, dim3(256), 0, stream, xi, o, rows, cols, index, count);
   return hipGetLastError();
 }
 
