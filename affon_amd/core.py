@@ -22,6 +22,7 @@ from __future__ import annotations
 
 import ctypes
 import itertools
+import math
 import weakref
 from dataclasses import dataclass
 from typing import Any, Callable, Mapping, Sequence
@@ -126,10 +127,9 @@ class Tensor:
         self.strides = tuple(int(s) for s in strides)
         self.offset = int(offset_elements)
         self._disposed = False
-
-    @property
-    def spec(self) -> TensorSpec:
-        return TensorSpec(self.dtype, self.shape)
+        # What every call on the tensor asks for; a tensor's description never changes.
+        self.spec = TensorSpec(self.dtype, self.shape)
+        self._view: _native.View | None = None
 
     def _check_live(self) -> None:
         if self._disposed or self._buffer.ptr is None:
@@ -137,11 +137,13 @@ class Tensor:
 
     def view(self) -> _native.View:
         self._check_live()
-        if len(self.shape) != 2 or self.dtype not in _NATIVE_DTYPE:
-            raise TypeError("rank-two f32/bf16/u32 tensor required")
-        return _native.View(self._buffer.ptr, self._buffer.nbytes, self.offset * _ITEMSIZE[self.dtype],
-                            (ctypes.c_int64 * 2)(*self.shape), (ctypes.c_int64 * 2)(*self.strides),
-                            _NATIVE_DTYPE[self.dtype])
+        if self._view is None:
+            if len(self.shape) != 2 or self.dtype not in _NATIVE_DTYPE:
+                raise TypeError("rank-two f32/bf16/u32 tensor required")
+            self._view = _native.View(self._buffer.ptr, self._buffer.nbytes, self.offset * _ITEMSIZE[self.dtype],
+                                      (ctypes.c_int64 * 2)(*self.shape), (ctypes.c_int64 * 2)(*self.strides),
+                                      _NATIVE_DTYPE[self.dtype])
+        return self._view
 
     @property
     def data_ptr(self) -> int:
@@ -216,9 +218,8 @@ class Session:
         if dtype not in DTYPES:
             raise TypeError(f"unsupported dtype: {dtype}")
         shape = tuple(int(d) for d in shape)
-        count = int(np.prod(shape)) if shape else 1
-        strides = tuple(int(np.prod(shape[i + 1:])) for i in range(len(shape)))
-        return Tensor(self, _Buffer(self, count * _ITEMSIZE[dtype]), dtype, shape, strides)
+        strides = tuple(math.prod(shape[i + 1:]) for i in range(len(shape)))
+        return Tensor(self, _Buffer(self, math.prod(shape) * _ITEMSIZE[dtype]), dtype, shape, strides)
 
     def tensor(self, values: Any, dtype: str = "f32") -> Tensor:
         """Creates a device tensor from host values (nested lists or arrays)."""

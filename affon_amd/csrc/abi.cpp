@@ -11,25 +11,167 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <exception>
 #include <limits>
+#include <map>
 #include <mutex>
 #include <string>
-#include <unordered_set>
+#include <unordered_map>
 #include <vector>
 
 #include "affon_rocm.h"
 #include "internal.h"
 
+// Device memory of a session. A freed block is kept for a later allocation of
+// its size class instead of going back to the runtime: hipMalloc and hipFree
+// cost tens of microseconds to milliseconds (a dequantize to 117 MB took 3.3
+// ms in a loop for 36 us of kernel), and every free waited for the stream.
+//
+// What hipFree gave stays: memory is handed out again only when nothing
+// anywhere on the device can still use it. A freed block waits in `resting`
+// until the device has been idle at some moment after its free, whatever
+// streams the caller used it on; blocks of one class are allocated anew
+// until kRest of them rest, so that the wait comes once for many frees.
+// At most kKeepBytes are kept, blocks over kMostBytes not at all; the rest
+// goes back to the runtime, as everything does when an allocation fails and
+// when the session ends.
+//
+// alloc and free may come from any thread (a caller's garbage collector
+// frees from whichever thread it runs on): the mutex guards everything.
+class DeviceMemory {
+ public:
+  explicit DeviceMemory(hipStream_t stream) : stream_(stream) {}
+
+  hipError_t alloc(size_t bytes, void** out) {
+    const size_t size = bytes <= kMostBytes ? size_class(bytes) : bytes;
+    std::lock_guard<std::mutex> lock(mutex_);
+    auto ready = ready_.find(size);
+    if (ready == ready_.end() && worth_a_wait(size) && settle()) ready = ready_.find(size);
+    if (ready != ready_.end()) {
+      *out = ready->second.back();
+      ready->second.pop_back();
+      if (ready->second.empty()) ready_.erase(ready);
+      kept_ -= size;
+    } else {
+      hipError_t e = hipMalloc(out, size);
+      if (e != hipSuccess && kept_ > 0) {
+        (void)hipGetLastError();
+        give_back();
+        e = hipMalloc(out, size);
+      }
+      if (e != hipSuccess) {
+        (void)hipGetLastError();
+        *out = nullptr;
+        return e;
+      }
+    }
+    owned_.emplace(*out, size);
+    return hipSuccess;
+  }
+
+  // False when this session did not allocate ptr.
+  bool free(void* ptr, hipError_t* status) {
+    *status = hipSuccess;
+    std::lock_guard<std::mutex> lock(mutex_);
+    const auto it = owned_.find(ptr);
+    if (it == owned_.end()) return false;
+    const size_t size = it->second;
+    owned_.erase(it);
+    if (size <= kMostBytes) {
+      if (kept_ + size > kKeepBytes) give_back();
+      resting_.push_back({size, ptr});
+      ++resting_classes_[size];
+      kept_ += size;
+      return true;
+    }
+    *status = hipStreamSynchronize(stream_);
+    const hipError_t e = hipFree(ptr);
+    if (*status == hipSuccess) *status = e;
+    return true;
+  }
+
+  // Everything, live allocations too (the session's work has ended).
+  void release_all() {
+    std::lock_guard<std::mutex> lock(mutex_);
+    give_back();
+    for (const auto& block : owned_) (void)hipFree(block.first);
+    owned_.clear();
+  }
+
+ private:
+  static constexpr size_t kKeepBytes = size_t(1) << 30;
+  static constexpr size_t kMostBytes = size_t(256) << 20;
+  static constexpr size_t kRest = 16;
+
+  // Sizes round up to eighths of a power of two, at least 256 bytes.
+  static size_t size_class(size_t bytes) {
+    size_t unit = 256;
+    while (unit * 16 < bytes) unit *= 2;
+    return (bytes + unit - 1) / unit * unit + (bytes == 0 ? unit : 0);
+  }
+  bool capturing() const {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    const hipError_t e = hipStreamIsCapturing(stream_, &capture);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e != hipSuccess || capture != hipStreamCaptureStatusNone;
+  }
+  // Whether a resting block of this class is worth waiting for the device:
+  // kRest of them rest (of a large class, half of what is kept), or the
+  // session's own work is done, so that there is hardly anything to wait for.
+  bool worth_a_wait(size_t size) const {
+    const auto it = resting_classes_.find(size);
+    if (it == resting_classes_.end()) return false;
+    if (it->second >= kRest || it->second * size >= kKeepBytes / 2) return true;
+    if (capturing()) return false;
+    const hipError_t e = hipStreamQuery(stream_);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e == hipSuccess;
+  }
+  // Waits for the device and makes the resting blocks ready; false (nothing
+  // changed) where it cannot wait now, as while the stream is captured.
+  bool settle() {
+    if (capturing()) return false;
+    if (hipDeviceSynchronize() != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    for (const Block& b : resting_) ready_[b.size].push_back(b.ptr);
+    resting_.clear();
+    resting_classes_.clear();
+    return true;
+  }
+  // Returns every kept block to the runtime, which waits for its users too.
+  void give_back() {
+    if (!resting_.empty()) (void)settle();
+    for (const Block& b : resting_) (void)hipFree(b.ptr);
+    for (const auto& entry : ready_)
+      for (void* ptr : entry.second) (void)hipFree(ptr);
+    resting_.clear();
+    resting_classes_.clear();
+    ready_.clear();
+    kept_ = 0;
+  }
+
+  struct Block {
+    size_t size;
+    void* ptr;
+  };
+  hipStream_t stream_;
+  std::mutex mutex_;
+  std::unordered_map<void*, size_t> owned_;  // handed out: size class by address
+  std::map<size_t, std::vector<void*>> ready_;
+  std::vector<Block> resting_;
+  std::unordered_map<size_t, size_t> resting_classes_;
+  size_t kept_ = 0;  // bytes of ready_ and resting_
+};
+
 struct affon_rocm_session {
   int device = 0;
   hipStream_t stream = nullptr;
   affon::Workspace* workspace = nullptr;
-  // Allocations made through affon_rocm_alloc and not yet freed: the
-  // session frees them when it ends, so tensors that outlive it leak nothing.
-  // alloc and free may come from any thread (a caller's garbage collector
-  // frees from whichever thread it runs on): the mutex guards the set.
-  std::mutex allocations_mutex;
-  std::unordered_set<void*> allocations;
+  // Allocations made through affon_rocm_alloc; the session frees those still
+  // live when it ends, so tensors that outlive it leak nothing.
+  DeviceMemory* memory = nullptr;
 };
 
 namespace affon {
@@ -332,6 +474,7 @@ int affon_rocm_session_create(int device, affon_rocm_session** out) {
   session->device = device;
   session->stream = stream;
   session->workspace = new affon::Workspace(device, stream);
+  session->memory = new DeviceMemory(stream);
   *out = session;
   return AFFON_ROCM_OK;
 }
@@ -343,17 +486,14 @@ int affon_rocm_session_destroy(affon_rocm_session* session) {
   if (hipSetDevice(session->device) == hipSuccess && session->stream != nullptr) {
     hipError_t e = hipStreamSynchronize(session->stream);
     if (e != hipSuccess) status = hip_fail(e, "hipStreamSynchronize");
-    {
-      std::lock_guard<std::mutex> lock(session->allocations_mutex);
-      for (void* ptr : session->allocations) (void)hipFree(ptr);
-      session->allocations.clear();
-    }
+    session->memory->release_all();
     delete session->workspace;
     e = hipStreamDestroy(session->stream);
     if (e != hipSuccess && status == AFFON_ROCM_OK) status = hip_fail(e, "hipStreamDestroy");
   } else {
     delete session->workspace;
   }
+  delete session->memory;
   delete session;
   return status;
 }
@@ -368,10 +508,12 @@ int affon_rocm_alloc(affon_rocm_session* session, size_t bytes, void** out) {
   if (status != AFFON_ROCM_OK) return status;
   if (out == nullptr) return fail(AFFON_ROCM_CORE_FAILURE, "allocation output is null");
   *out = nullptr;
-  hipError_t e = hipMalloc(out, bytes == 0 ? 1 : bytes);
-  if (e != hipSuccess) return hip_fail(e, "hipMalloc");
-  std::lock_guard<std::mutex> lock(session->allocations_mutex);
-  session->allocations.insert(*out);
+  try {
+    const hipError_t e = session->memory->alloc(bytes, out);
+    if (e != hipSuccess) return hip_fail(e, "hipMalloc");
+  } catch (const std::exception& e) {
+    return fail(AFFON_ROCM_CORE_FAILURE, "alloc: %s", e.what());
+  }
   return AFFON_ROCM_OK;
 }
 
@@ -380,14 +522,13 @@ int affon_rocm_free(affon_rocm_session* session, void* ptr) {
   int status = check_session(session);
   if (status != AFFON_ROCM_OK) return status;
   if (ptr == nullptr) return AFFON_ROCM_OK;
-  {
-    std::lock_guard<std::mutex> lock(session->allocations_mutex);
-    if (session->allocations.erase(ptr) == 0)
+  hipError_t e = hipSuccess;
+  try {
+    if (!session->memory->free(ptr, &e))
       return fail(AFFON_ROCM_CORE_FAILURE, "free of memory this session did not allocate");
+  } catch (const std::exception& error) {
+    return fail(AFFON_ROCM_CORE_FAILURE, "free: %s", error.what());
   }
-  hipError_t e = hipStreamSynchronize(session->stream);
-  if (e != hipSuccess) return hip_fail(e, "hipStreamSynchronize");
-  e = hipFree(ptr);
   if (e != hipSuccess) return hip_fail(e, "hipFree");
   return AFFON_ROCM_OK;
 }
@@ -947,10 +1088,7 @@ struct DeviceBuffer {
   void* ptr = nullptr;
   explicit DeviceBuffer(affon_rocm_session* s) : session(s) {}
   ~DeviceBuffer() {
-    if (ptr != nullptr) {
-      hipSetDevice(session->device);
-      hipFree(ptr);
-    }
+    if (ptr != nullptr) (void)affon_rocm_free(session, ptr);
   }
 };
 

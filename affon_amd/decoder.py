@@ -181,12 +181,8 @@ class QuantizedDecoderBlock:
     # ---- running ----
 
     def _run(self, source: Program, inputs: Mapping[str, Tensor], **options):
-        executable = self.session.compile(source, **options)
-        arguments = self.weight_arguments()
-        needed = {n["name"] for n in source.nodes if n["kind"] == "argument"}
-        arguments = {k: v for k, v in arguments.items() if k in needed}
-        arguments.update(inputs)
-        return executable.run(arguments)
+        # run() reads the arguments its Program names.
+        return self.session.compile(source, **options).run({**self.weight_arguments(), **inputs})
 
     def attention(self, normalized: Tensor, **options) -> list[Tensor]:
         """(query, key, value) of normalized activations [M, width]."""

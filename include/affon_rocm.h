@@ -102,6 +102,11 @@ int affon_rocm_session_destroy(affon_rocm_session* session);
 /* The session's hipStream_t, for callers that record events around its work. */
 void* affon_rocm_session_stream(affon_rocm_session* session);
 
+/* Device memory of the session. Freed memory is kept for later allocations of
+ * the session (at most 1 GiB, no block over 256 MiB) and handed out again only
+ * after the device has been idle since its free, as a return to the runtime
+ * would wait for; a free does not wait. It goes back to the runtime when an
+ * allocation fails for want of it and when the session ends. */
 int affon_rocm_alloc(affon_rocm_session* session, size_t bytes, void** out);
 int affon_rocm_free(affon_rocm_session* session, void* ptr);
 /* Copies are ordered on the session stream and complete before returning. */

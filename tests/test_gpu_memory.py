@@ -1,0 +1,93 @@
+"""GPU: memory that a session keeps between allocations is bounded, is handed
+out again only when nothing can still use it, and is given back."""
+import ctypes
+import gc
+import threading
+
+import numpy as np
+import pytest
+
+import affon_amd as A
+from affon_amd import _native
+from tests.helpers import HipRuntime
+
+pytestmark = pytest.mark.gpu
+MIB = 1 << 20
+
+
+def raw_alloc(session, nbytes):
+    ptr = ctypes.c_void_p()
+    _native.check(_native.load().affon_rocm_alloc(session._handle, nbytes, ctypes.byref(ptr)), "alloc")
+    return ptr.value
+
+
+def test_kept_memory_is_bounded_and_given_back():
+    hip = HipRuntime()
+    with A.Session("rocm") as session:
+        lib = _native.load()
+        before = hip.free_bytes()
+        for size in (200 * MIB, 120 * MIB, 300 * MIB, 7 * MIB):  # 300 MiB: over what is kept
+            blocks = [raw_alloc(session, size) for _ in range(6)]
+            assert len(set(blocks)) == 6
+            for b in blocks:
+                assert lib.affon_rocm_free(session._handle, b) == 0
+            assert hip.free_bytes() >= before - 1100 * MIB, size
+        # Freed once: not this session's any more, whether kept or not.
+        assert lib.affon_rocm_free(session._handle, blocks[0]) == _native.CORE_FAILURE
+    assert hip.free_bytes() >= before - 64 * MIB
+
+
+def test_memory_comes_back_only_when_idle(session, rng):
+    """Results whose tensors die while later work still runs keep their
+    values as long as they are held: a loop of products, each result dropped
+    two rounds later, against the first round's."""
+    x = session.tensor(rng.standard_normal((64, 4096)).astype(np.float32))
+    w = A.quantize(session.tensor(rng.standard_normal((4096, 4096)).astype(np.float32)), bits=4, group_size=64,
+                   param_dtype="f32")
+    want = A.quantized_matmul(x, *w, bits=4, group_size=64).numpy()
+    recent = []
+    for i in range(60):
+        recent.append(A.quantized_matmul(x, *w, bits=4, group_size=64))
+        if len(recent) > 2:
+            recent.pop(0)
+        if i % 20 == 19:
+            for t in recent:
+                np.testing.assert_array_equal(t.numpy(), want)
+
+
+def test_frees_from_other_threads(session):
+    """Tensors dropped on other threads while this one allocates: addresses of
+    live tensors never coincide, and their contents stay."""
+    stop, errors = threading.Event(), []
+    dropped = []
+
+    def drop():
+        while not stop.is_set():
+            try:
+                dropped.pop(0)
+            except IndexError:
+                pass
+            except Exception as e:  # noqa: BLE001 - reported below
+                errors.append(e)
+
+    threads = [threading.Thread(target=drop) for _ in range(2)]
+    for t in threads:
+        t.start()
+    try:
+        live = []
+        for i in range(400):
+            t = session.tensor(np.full(1000 + i % 3, i, np.float32))
+            live.append((i, t))
+            assert len({v._buffer.ptr for _, v in live}) == len(live)
+            if len(live) > 8:
+                j, old = live.pop(0)
+                assert (old.numpy() == j).all()
+                dropped.append(old)
+                del old
+    finally:
+        stop.set()
+        for t in threads:
+            t.join()
+        dropped.clear()
+        gc.collect()
+    assert not errors
