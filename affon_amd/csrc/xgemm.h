@@ -12,10 +12,11 @@
 // exact in f32, and each run of 64 k (32 where groups are not multiples of
 // 64) adds s * sum(x*q) + b * sum(x) in f32, as the VALU decode kernel does
 // per 16 bytes of codes: the run's term is formed first and added
-// to the output's sum once, and with bf16 activations, whose terms carry next
-// to no rounding, a sum of kRunSteps steps is then added to its total (one
-// chain with two roundings per run put 100 x 4096 x 1376 at groups of 32 from
-// 7.3e-8 off 64 bits to 1.0e-7; f32 activations: 2.8e-7 before, 2.0e-7 here,
+// to the output's sum once, and with bf16 activations, whose products carry next
+// to no rounding, a sum of kRunSteps steps is then added to its total and the
+// codes count from the middle of their range (centred_start; 100 x 4096 x 1376
+// at groups of 32, off 64 bits: 7.3e-8 on the VALU kernel, 1.0e-7 in one chain
+// with two roundings per run, 8.2e-8 with runs alone, 7.0e-8 with both; f32 activations: 2.8e-7 before, 2.0e-7 here,
 // most of it the terms' own). The small planes accumulate first.
 //
 // Two kernels:
@@ -69,6 +70,30 @@ template <typename XT>
 constexpr int kPlanes = XT::bytes == 4 ? 3 : 1;
 
 constexpr int kRunSteps = 8;  // a power of two
+
+// bf16 activations: codes count from the middle of their range, c = 2^(BITS-1),
+//   s * sum(x*q) + b * sum(x) = s * (sum(x*q) - c * sum(x)) + (b + c*s) * sum(x).
+// The bias of a group lies near its least value, so that the two terms on the
+// left are each two to three times their sum, and their roundings most of the
+// error; on the right the second is small. The products start from
+// -c * sum(x) instead of zero, which costs no instruction per output. (With
+// f32 activations the chain starts with the small planes, which that start
+// would round.)
+template <typename XT>
+constexpr bool kCentred = XT::bytes == 2;
+template <int BITS>
+constexpr float kCentre = static_cast<float>(1 << (BITS - 1));
+// What a run's products start from. Zero where the sum is infinite or NaN, so
+// that an infinite activation does not meet its own negative there.
+template <int BITS>
+__device__ __forceinline__ float centred_start(float sum) {
+  const float v = -kCentre<BITS> * sum;
+  return fabsf(v) < INFINITY ? v : 0.0f;
+}
+template <int BITS, typename XT>
+__device__ __forceinline__ float centred_bias(float s, float b) {
+  return kCentred<XT> ? fmaf(kCentre<BITS>, s, b) : b;
+}
 
 // Eight consecutive activations as loaded.
 template <typename XT>
@@ -403,6 +428,14 @@ __global__ __launch_bounds__(kThreads, 2) void xskinny_kernel(Args args) {
               xs[rb][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, xp[rb][t][p]), ones,
                                                                   xs[rb][i], 0, 0, 0);
         }
+      f32x4_t start[RB][kBlocks];
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int i = 0; i < kBlocks; ++i)
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+            start[rb][i][v] = kCentred<XT> ? centred_start<BITS>(xs[rb][i][v]) : 0.0f;
       // Two column tiles at a time: their product chains are independent.
 #pragma unroll
       for (int c0 = 0; c0 < 4; c0 += 2) {
@@ -441,11 +474,12 @@ __global__ __launch_bounds__(kThreads, 2) void xskinny_kernel(Args args) {
                 for (int c = 0; c < 2; ++c)
                   q[rb][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                       __builtin_bit_cast(bf16x8_t, xp[rb][t][p]), __builtin_bit_cast(bf16x8_t, op[c][t]),
-                      p == P - 1 && t == (G32 ? i : 0) ? f32x4_t{0.0f, 0.0f, 0.0f, 0.0f} : q[rb][c], 0, 0, 0);
+                      p == P - 1 && t == (G32 ? i : 0) ? start[rb][i] : q[rb][c], 0, 0, 0);
 #pragma unroll
           for (int c = 0; c < 2; ++c) {
             const int at = (16 * (c0 + c) + r) * kWindowBytes<PT>;
-            float sv = param_at<PT>(own_s + at, g[i] - window), bv = param_at<PT>(own_b + at, g[i] - window);
+            float sv = param_at<PT>(own_s + at, g[i] - window);
+            float bv = centred_bias<BITS, XT>(sv, param_at<PT>(own_b + at, g[i] - window));
             if (step * kBK + 32 * i >= a.K) sv = bv = 0.0f;  // past the end of K
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb)
@@ -517,6 +551,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void xtile_kernel(Args args) {
   static_assert(BM * 8 % kTileThreads == 0, "whole chunks per thread");
   __shared__ __attribute__((aligned(16))) uint8_t lds_x[2][P][BM * 128];
   __shared__ __attribute__((aligned(16))) float lds_sum[2][kBlocks][BM];
+  __shared__ __attribute__((aligned(16))) float lds_start[kCentred<XT> ? 2 : 1][kBlocks][kCentred<XT> ? BM : 1];
   __shared__ __attribute__((aligned(16))) uint8_t lds_p[2][2][BN * kWindowBytes<PT>];  // [window][scale, bias]
   static_assert(kTileThreads >= 2 * BN, "a thread per column and parameter");
 
@@ -559,7 +594,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void xtile_kernel(Args args) {
 #pragma unroll
     for (int p = 0; p < P; ++p) *reinterpret_cast<u32x4_t*>(&lds_x[stage][p][slot(row, sq)]) = pl[p];
     const float sum = run_sum<G32>(part_sum);
-    if ((sq & (G32 ? 3 : 7)) == 0) lds_sum[stage][G32 ? sq >> 2 : 0][row] = sum;
+    if ((sq & (G32 ? 3 : 7)) == 0) {
+      lds_sum[stage][G32 ? sq >> 2 : 0][row] = sum;
+      if constexpr (kCentred<XT>) lds_start[stage][G32 ? sq >> 2 : 0][row] = centred_start<BITS>(sum);
+    }
   };
 
   // Packed words of a step: two runs of 16 codes per column, run j holding
@@ -682,7 +720,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void xtile_kernel(Args args) {
         const int col = (32 * (CT * ni + ct) + li) * kWindowBytes<PT>;
         const uint32_t g = args.group_of(2 * t + i) - (latest ? window[1] : window[0]);
         sv[ct][i] = param_at<PT>(&lds_p[latest][0][col], g);
-        bv[ct][i] = param_at<PT>(&lds_p[latest][1][col], g);
+        bv[ct][i] = centred_bias<BITS, XT>(sv[ct][i], param_at<PT>(&lds_p[latest][1][col], g));
         if (i == 1 && t * kBK + 32 >= a.K) sv[ct][i] = bv[ct][i] = 0.0f;  // past the end of K
       }
     }
@@ -699,7 +737,15 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void xtile_kernel(Args args) {
       f32x16_t term[CT];
 #pragma unroll
       for (int i = 0; i < kBlocks; ++i) {
-        f32x16_t acc[CT];
+        f32x16_t acc[CT], start = zero;
+        if constexpr (kCentred<XT>) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const f32x4_t v = *reinterpret_cast<const f32x4_t*>(&lds_start[stage][i][row0 + 8 * u + 4 * lh]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) start[4 * u + e] = v[e];
+          }
+        }
 #pragma unroll
         for (int p = P - 1; p >= 0; --p)
 #pragma unroll
@@ -709,7 +755,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void xtile_kernel(Args args) {
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct)
               acc[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf, __builtin_bit_cast(bf16x8_t, op[ct][kPart * i + kk]),
-                                                                p == P - 1 && kk == 0 ? zero : acc[ct], 0, 0, 0);
+                                                                p == P - 1 && kk == 0 ? (kCentred<XT> ? start : zero) : acc[ct], 0, 0, 0);
           }
         // Accumulator element v of lane l: row 8*(v/4) + 4*(l/32) + v%4, column l%32.
         f32x4_t xs[4];

@@ -143,3 +143,22 @@ def test_capture_without_scratch(M, rng):
                 A.quantized_matmul(*t, bits=8, group_size=group)
         finally:
             hip.destroy(graph)
+
+
+@pytest.mark.parametrize("M", [3, 40, 200])
+@pytest.mark.parametrize("bits", [2, 4, 8])
+def test_bf16_products_start_from_their_sums(session, bits, M):
+    """bf16 activations: rows of one value, whose products and sums are all
+    exact, so that nothing of the start -2^(bits-1) * sum(x) may remain; an
+    infinite row stays infinite with positive scales and biases."""
+    N, K, group = 70, 320, 32
+    x = np.zeros((M, K), np.float32)
+    picked = np.array([1.5, -2.0 ** 60, np.inf, -np.inf, np.nan, 2.0 ** -100], np.float32)[np.arange(M) % 6]
+    x[np.arange(M), np.arange(M) * 7 % K] = picked
+    q = np.full((N, K), (1 << bits) - 1, np.int64)
+    s, b = np.full((N, K // group), 2.0 ** -10, np.float32), np.full((N, K // group), 0.25, np.float32)
+    t = upload_all(session, storage(x, "bf16"), q, s, b, bits, "bf16", "f32")
+    out = session.empty("f32", (M, N))
+    A.quantized_matmul_into(out, *t, bits=bits, group_size=group, implementation="gemv")
+    want = picked * np.float32(q[0, 0] * 2.0 ** -10 + 0.25)
+    np.testing.assert_array_equal(out.numpy(), np.broadcast_to(want[:, None], (M, N)))
