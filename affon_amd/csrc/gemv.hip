@@ -315,14 +315,26 @@ hipError_t gemv_group_launch(const QmmProblem* group, int count, const Launch& l
 }
 
 namespace {
-// Up to four rows cost this file's kernel one pass over the weights. Where
-// its decode is cheap (8-bit codes; 2-bit codes a word at a time) and the
+// This file's kernel passes over the weights once per four rows. Where its
+// decode is cheap (8-bit codes; 2-bit codes a word at a time) and the
 // matrix-core kernel would have to split K to fill the GPU, which costs a
-// second launch, the one pass is ahead: 2 x 4096 x 4096 f32 at 8 bits 12.0
-// against 15.5 us, 2-bit groups of 32 2 x 4096 x 4160 11.8 against 16.1; from
-// 128 column tiles on it is behind (14336 columns: 30.2 against 20.9).
-bool one_pass_is_ahead(const QmmProblem& p) {
-  return p.M <= 4 && p.N <= 8192 && (p.bits == 8 || (p.bits == 2 && p.group % 64 != 0));
+// second launch, few passes over few columns are ahead. In us a call, this
+// kernel first, f32 at 8 bits and K = 4096: 2 x 4096 11.4 and 12.6, 8 x 1024
+// 8.7 and 11.2, 16 x 1024 11.3 and 11.8, 8 x 4096 20.5 and 13.4; 2-bit groups
+// of 32 2 x 4096 x 4160 11.8 and 16.1, 15 x 423 x 2624 11.3 and 14.7; from 128
+// column tiles on it is behind (14336 columns: 30.2 and 20.9). A long K leaves
+// few columns' waves too much each: K = 14336 4 x 256 15.9 and 12.4, 4 x 1024
+// 16.4 and 14.6, but 2 x 4096 21.6 and 24.5. With bf16 activations 4-bit codes
+// are a little ahead too: 2 x 1024 x 4128 9.8 and 11.0, 8 x 1024 10.5 and 11.4
+// (K = 1376, where the other needs no ranges: 9.5 and 7.9; 16 x 1024 19.2 and
+// 11.7).
+bool few_passes_are_ahead(const QmmProblem& p) {
+  const int64_t columns = (p.M + 3) / 4 * p.N;  // over all passes
+  if (p.bits == 4) return p.x_dtype == AFFON_ROCM_BF16 && columns <= 2048 && p.K > 2048 && p.K <= 8192;
+  const bool two_bit_words = p.bits == 2 && p.group % 64 != 0;
+  if (p.bits == 2 && !two_bit_words) return false;
+  if (p.M <= 4) return p.N <= 8192 && (p.N > 2048 || p.K <= 8192 || two_bit_words);
+  return columns <= 4096 && p.K <= 8192;
 }
 }  // namespace
 
@@ -336,7 +348,7 @@ hipError_t gemv_launch(const QmmProblem& p, const Launch& l) {
       default: return gemv1_launch_b8(p, stream);
     }
   }
-  if (!one_pass_is_ahead(p) && xgemm_supports(p)) return xgemm_launch(p, l);
+  if (!few_passes_are_ahead(p) && xgemm_supports(p)) return xgemm_launch(p, l);
   switch (p.bits) {
     case 2: return launch_bits<2>(p, stream);
     case 4: return launch_bits<4>(p, stream);

@@ -14,10 +14,11 @@
 // per 16 bytes of codes: the run's term is formed first and added
 // to the output's sum once, and with bf16 activations, whose products carry next
 // to no rounding, a sum of kRunSteps steps is then added to its total and the
-// codes count from the middle of their range (centred_start; 100 x 4096 x 1376
+// codes count from the middle of their range (centred_start). 100 x 4096 x 1376
 // at groups of 32, off 64 bits: 7.3e-8 on the VALU kernel, 1.0e-7 in one chain
-// with two roundings per run, 8.2e-8 with runs alone, 7.0e-8 with both; f32 activations: 2.8e-7 before, 2.0e-7 here,
-// most of it the terms' own). The small planes accumulate first.
+// with two roundings per run, 8.2e-8 with runs alone, 7.0e-8 with both. f32
+// activations: 2.8e-7 before, 2.0e-7 here, most of it the terms' own; the
+// small planes accumulate first.
 //
 // Two kernels:
 //   xskinny  up to 32 rows: each wave of a 64-column workgroup walks a K part

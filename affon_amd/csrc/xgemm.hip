@@ -14,7 +14,9 @@ hipError_t launch_b8(const Args& args, Shape shape, bool g32, int x_dtype, int p
 namespace {
 
 constexpr int64_t kMaxPartialBytes = int64_t(32) << 20;  // what the no-allocation entry point holds
-constexpr int kMaxSplits = 8;
+// Few columns and a long K: with eight ranges 48 x 256 x 14336 takes 38 us a
+// call, with 16 24.2 and with 32 18.1; the reduction reads eight at a time.
+constexpr int kMaxSplits = 32;
 
 int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 

@@ -162,3 +162,32 @@ def test_bf16_products_start_from_their_sums(session, bits, M):
     A.quantized_matmul_into(out, *t, bits=bits, group_size=group, implementation="gemv")
     want = picked * np.float32(q[0, 0] * 2.0 ** -10 + 0.25)
     np.testing.assert_array_equal(out.numpy(), np.broadcast_to(want[:, None], (M, N)))
+
+
+@pytest.mark.parametrize("M,N", [(1, 1), (3, 1), (1, 3), (33, 1), (35, 3), (33, 67), (40, 64)])
+def test_reductions_of_many_ranges(session, M, N, rng):
+    """32 K ranges and their ordered sum, for counts of outputs below four and
+    of every remainder by four."""
+    K, bits, group = 8192, 8, 64
+    x, q, s, b = operands(rng, M, N, K, bits, group, "f32", "f32")
+    t = upload_all(session, x, q, s, b, bits, "f32", "f32")
+    out = session.tensor(np.full((M, N), np.nan, np.float32))
+    A.quantized_matmul_into(out, *t, bits=bits, group_size=group, implementation="gemv")
+    want, bound = expected_and_bound(x, q, s, b, group)
+    err = np.abs(out.numpy() - want)
+    assert (err <= bound).all() and np.linalg.norm(err) <= 2e-6 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("bits,group,x_dtype,K", [(8, 64, "f32", 8192), (8, 64, "f32", 8256), (2, 32, "bf16", 2624),
+                                                  (4, 32, "bf16", 2048), (4, 32, "bf16", 2080), (4, 32, "bf16", 8224)])
+def test_sides_of_the_few_passes_rule(session, bits, group, x_dtype, K, rng):
+    """Rows and columns on both sides of the lines between the VALU and the
+    matrix-core kernels."""
+    for M, N in ((2, 70), (4, 2048), (5, 1024), (5, 1025), (8, 2048), (8, 2049)):
+        x, q, s, b = operands(rng, M, N, K, bits, group, x_dtype, "bf16")
+        t = upload_all(session, x, q, s, b, bits, x_dtype, "bf16")
+        out = session.tensor(np.full((M, N), np.nan, np.float32))
+        A.quantized_matmul_into(out, *t, bits=bits, group_size=group, implementation="gemv")
+        want, bound = expected_and_bound(x, q, s, b, group)
+        err = np.abs(out.numpy() - want)
+        assert (err <= bound).all() and np.linalg.norm(err) <= 2e-6 * np.linalg.norm(want), (M, N)
