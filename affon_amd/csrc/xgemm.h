@@ -80,16 +80,18 @@ constexpr int kRunSteps = 8;  // a power of two
 // -c * sum(x) instead of zero, which costs no instruction per output. (With
 // f32 activations the chain starts with the small planes, which that start
 // would round.)
+// The right side overflows sooner (in c * sum(x) and c * s), and an infinite x
+// meets its own negative in it. What has overflowed is never finite again, so
+// that finite outputs are right; the others are computed again as on the left
+// (plain_sum). That is after the loop, for no registers or instructions in it.
 template <typename XT>
 constexpr bool kCentred = XT::bytes == 2;
 template <int BITS>
 constexpr float kCentre = static_cast<float>(1 << (BITS - 1));
-// What a run's products start from. Zero where the sum is infinite or NaN, so
-// that an infinite activation does not meet its own negative there.
+// What a run's products start from.
 template <int BITS>
 __device__ __forceinline__ float centred_start(float sum) {
-  const float v = -kCentre<BITS> * sum;
-  return fabsf(v) < INFINITY ? v : 0.0f;
+  return -kCentre<BITS> * sum;
 }
 template <int BITS, typename XT>
 __device__ __forceinline__ float centred_bias(float s, float b) {
@@ -230,6 +232,41 @@ __device__ __forceinline__ float run_sum(float v) {
 template <typename XT>
 __device__ __forceinline__ float sum8(const Raw8<XT>& v) {
   return ((v.at(0) + v.at(1)) + (v.at(2) + v.at(3))) + ((v.at(4) + v.at(5)) + (v.at(6) + v.at(7)));
+}
+
+// One output's sum over K steps [step, end) as s * sum(x*q) + b * sum(x) per 32
+// values, until it is a NaN: one thread to an output, for those that the
+// centred form overflows in. 4-bit groups of 32, 16 x 4096 x 1376 and 512 rows:
+// 9.4 and 32 us a call of ordinary values, 18 and 44 of NaNs alone, 94 and 446
+// where every output is infinite and stays so (VALU kernel 66 and 2090).
+template <int BITS, typename XT, typename PT>
+__device__ __forceinline__ float plain_sum(const Args& args, int row, int col, int step, int end) {
+  const TileArgs& a = args.t;
+  const uint8_t* x = reinterpret_cast<const uint8_t*>(a.x) + static_cast<int64_t>(row) * a.xs0 * XT::bytes;
+  const uint32_t* w = a.w + static_cast<int64_t>(col) * a.ws0;
+  const uint8_t* s = a.s + static_cast<int64_t>(col) * a.ss0 * PT::bytes;
+  const uint8_t* b = a.b + static_cast<int64_t>(col) * a.bs0 * PT::bytes;
+  const int blocks = min(2 * end, a.K / 32);
+  float total = 0.0f;
+#pragma unroll 1
+  for (int i = 2 * step; i < blocks && total == total; ++i) {
+    const uint32_t g = args.group_of(i);
+    Raw8<XT> v[4];
+    uint32_t word[BITS];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j].load(x + (static_cast<int64_t>(i) * 32 + 8 * j) * XT::bytes);
+#pragma unroll
+    for (int j = 0; j < BITS; ++j) word[j] = w[static_cast<int64_t>(i) * BITS + j];
+    float xq = 0.0f, xs = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 32; ++e) {
+      const uint32_t code = word[e * BITS / 32] >> (e * BITS % 32) & ((1u << BITS) - 1);
+      xq = fmaf(v[e / 8].at(e % 8), static_cast<float>(code), xq);
+      xs += v[e / 8].at(e % 8);
+    }
+    total += fmaf(PT::load(s, g), xq, PT::load(b, g) * xs);
+  }
+  return total;
 }
 
 // ---- up to 32 rows ---------------------------------------------------------
@@ -514,8 +551,28 @@ __global__ __launch_bounds__(kThreads, 2) void xskinny_kernel(Args args) {
 #pragma unroll
     for (int ct = 0; ct < 4; ++ct)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) ysum(wave)[ypos(16 * rb + 4 * h + v, 16 * ct + r)] =
-            kRuns ? total_y[rb][ct][v] + y[rb][ct][v] : y[rb][ct][v];
+      for (int v = 0; v < 4; ++v) {
+        if constexpr (kRuns) y[rb][ct][v] += total_y[rb][ct][v];
+        ysum(wave)[ypos(16 * rb + 4 * h + v, 16 * ct + r)] = y[rb][ct][v];
+      }
+  if constexpr (kCentred<XT>) {
+    bool overflow = false;
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int ct = 0; ct < 4; ++ct)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) overflow |= !(fabsf(y[rb][ct][v]) < INFINITY);
+    if (__any(overflow)) {
+      wave_order();
+#pragma unroll 1
+      for (int row = 0; row < min(kRows, a.M); ++row) {
+        float* sum = &ysum(wave)[ypos(row, lane)];
+        if (n0 + lane < a.N && !(fabsf(*sum) < INFINITY))
+          *sum = plain_sum<BITS, XT, PT>(args, row, n0 + lane, u0 * kSub, u1 * kSub);
+      }
+    }
+  }
   __syncthreads();
   float* dst = a.splits == 1 ? a.out : a.partial + split * static_cast<int64_t>(a.M) * a.N;
   with_store_kind(a.splits == 1 ? a.epi.kind : kEpiNone, [&](auto kind) {
@@ -789,20 +846,43 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void xtile_kernel(Args args) {
     if (t + 1 < t1) window_for(t + 1);
   }
 
+  // Element v of accumulator tile (rt, ct) is row row_of(rt, v) and column col_of(ct).
+  auto row_of = [&](int rt, int v) { return m0 + 32 * (RT * mi + rt) + 8 * (v / 4) + 4 * lh + v % 4; };
+  auto col_of = [&](int ct) { return n0 + 32 * (CT * ni + ct) + li; };
+  if constexpr (kCentred<XT>) {
+    static_assert(RT * CT * 16 <= 32, "a bit per output");
+    uint32_t overflow = 0;
+#pragma unroll
+    for (int i = 0; i < RT * CT * 16; ++i) {
+      y[i / 16 / CT][i / 16 % CT][i % 16] += total_y[i / 16 / CT][i / 16 % CT][i % 16];
+      overflow |= fabsf(y[i / 16 / CT][i / 16 % CT][i % 16]) < INFINITY ? 0u : 1u << i;
+    }
+    if (__any(overflow != 0)) {
+#pragma unroll 1
+      for (int i = 0; i < RT * CT * 16; ++i) {
+        const int row = row_of(i / 16 / CT, i % 16), col = col_of(i / 16 % CT);
+        if ((overflow >> i & 1) == 0 || row >= a.M || col >= a.N) continue;
+        const float sum = plain_sum<BITS, XT, PT>(args, row, col, t0, t1);
+#pragma unroll
+        for (int j = 0; j < RT * CT * 16; ++j)
+          y[j / 16 / CT][j / 16 % CT][j % 16] = j == i ? sum : y[j / 16 / CT][j / 16 % CT][j % 16];
+      }
+    }
+  }
+
   float* dst = a.splits == 1 ? a.out : a.partial + split * static_cast<int64_t>(a.M) * a.N;
   with_store_kind(a.splits == 1 ? a.epi.kind : kEpiNone, [&](auto kind) {
     constexpr int KIND = decltype(kind)::value;
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) {
-      const int col = n0 + 32 * (CT * ni + ct) + li;
+      const int col = col_of(ct);
       if (col < a.N) {
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
           for (int v = 0; v < 16; ++v) {
-            const int row = m0 + 32 * (RT * mi + rt) + 8 * (v / 4) + 4 * lh + v % 4;
-            if (row < a.M) store_as<KIND>(a.epi, dst + static_cast<int64_t>(row) * a.N + col, col,
-                                          kRuns ? total_y[rt][ct][v] + y[rt][ct][v] : y[rt][ct][v]);
+            const int row = row_of(rt, v);
+            if (row < a.M) store_as<KIND>(a.epi, dst + static_cast<int64_t>(row) * a.N + col, col, y[rt][ct][v]);
           }
       }
     }

@@ -191,3 +191,46 @@ def test_sides_of_the_few_passes_rule(session, bits, group, x_dtype, K, rng):
         want, bound = expected_and_bound(x, q, s, b, group)
         err = np.abs(out.numpy() - want)
         assert (err <= bound).all() and np.linalg.norm(err) <= 2e-6 * np.linalg.norm(want), (M, N)
+
+
+LOWEST_BF16 = -(2.0 ** 127) * (2 - 2.0 ** -7)
+
+
+@pytest.mark.parametrize("M,N,K", [(5, 2060, 352), (24, 1030, 352), (70, 1030, 352), (130, 2060, 16032)])
+@pytest.mark.parametrize("bits", [2, 4, 8])
+def test_large_bf16_activations(session, bits, M, N, K):
+    """Where 2^(bits-1) * sum(x) or a group's 2^(bits-1) * scale overflows, on
+    every kernel: one nonzero activation per row, negative, zero and positive
+    biases, codes on both sides of the middle. A result that f32 holds as
+    s * (q*x) + b*x lies within its terms' roundings; a row that is infinite
+    gives its true sign or, where the two terms' signs differ, a NaN; no row
+    changes another."""
+    group, c = 32, 2.0 ** (bits - 1)
+    picked = np.array([LOWEST_BF16, -LOWEST_BF16, 2.0 ** 121, -2.0 ** 122, 2.0 ** 123, 2.0 ** 124, -2.0 ** 125, 2.0 ** 126,
+                       np.inf, -np.inf, np.nan, 1.5, -2.0 ** 60])[np.arange(M) % 13]
+    at = np.arange(M) * 37 % K
+    x = np.zeros((M, K), np.float32)
+    x[np.arange(M), at] = picked
+    q = np.arange(N) % (1 << bits)  # a column's code
+    large = np.arange(N) % 5 == 4  # scales whose 2^(bits-1) times overflows at 8 bits
+    s = np.where(large, 2.0 ** 122, 2.0 ** -10)
+    b = s * np.where(large, 0.25, np.array([-(c - 0.5), 0.0, 0.25, -0.5 - c, c])[np.arange(N) // 3 % 5])
+    t = (session.from_bytes(storage(x, "bf16"), A.TensorSpec.bf16((M, K))),
+         session.from_bytes(np.repeat(pack_codes(np.repeat(q[:, None], 32 // bits, 1), bits), K * bits // 32, 1),
+                            A.TensorSpec.u32((N, K * bits // 32))),
+         *(session.from_bytes(storage(np.repeat(v[:, None], K // group, 1), "f32"), A.TensorSpec.f32((N, K // group)))
+           for v in (s, b)))
+    out = session.tensor(np.full((M, N), 7.0, np.float32))
+    A.quantized_matmul_into(out, *t, bits=bits, group_size=group, implementation="gemv")
+    got, v = out.numpy(), picked[:, None]
+    with np.errstate(over="ignore", invalid="ignore"):
+        qx, bx = (q * v).astype(np.float32), (b * v).astype(np.float32)
+        plain = s.astype(np.float32) * qx + bx
+        exact = (s * q + b) * v
+        bound = 4 * 2.0 ** -24 * (s * (q + 2 * c) + 2 * np.abs(b)) * np.abs(v)
+        held = np.isfinite(plain)
+        assert held.any() and (np.abs(got.astype(np.float64) - exact)[held] <= bound[held]).all()
+        infinite = np.isinf(v) & (s * q + b != 0)
+        assert (np.isnan(got) | (got == exact))[infinite].all()
+    assert (got == exact)[infinite & (b * q > 0)].all()  # both terms of one sign
+    assert np.isnan(got[np.isnan(picked)]).all()
