@@ -13,157 +13,12 @@
 #include <cstring>
 #include <exception>
 #include <limits>
-#include <map>
 #include <mutex>
 #include <string>
-#include <unordered_map>
 #include <vector>
 
 #include "affon_rocm.h"
 #include "internal.h"
-
-// Device memory of a session. A freed block is kept for a later allocation of
-// its size class instead of going back to the runtime: hipMalloc and hipFree
-// cost tens of microseconds to milliseconds (a dequantize to 117 MB took 3.3
-// ms in a loop for 36 us of kernel), and every free waited for the stream.
-//
-// What hipFree gave stays: memory is handed out again only when nothing
-// anywhere on the device can still use it. A freed block waits in `resting`
-// until the device has been idle at some moment after its free, whatever
-// streams the caller used it on; blocks of one class are allocated anew
-// until kRest of them rest, so that the wait comes once for many frees.
-// At most kKeepBytes are kept, blocks over kMostBytes not at all; the rest
-// goes back to the runtime, as everything does when an allocation fails and
-// when the session ends.
-//
-// alloc and free may come from any thread (a caller's garbage collector
-// frees from whichever thread it runs on): the mutex guards everything.
-class DeviceMemory {
- public:
-  explicit DeviceMemory(hipStream_t stream) : stream_(stream) {}
-
-  hipError_t alloc(size_t bytes, void** out) {
-    const size_t size = bytes <= kMostBytes ? size_class(bytes) : bytes;
-    std::lock_guard<std::mutex> lock(mutex_);
-    auto ready = ready_.find(size);
-    if (ready == ready_.end() && worth_a_wait(size) && settle()) ready = ready_.find(size);
-    if (ready != ready_.end()) {
-      *out = ready->second.back();
-      ready->second.pop_back();
-      if (ready->second.empty()) ready_.erase(ready);
-      kept_ -= size;
-    } else {
-      hipError_t e = hipMalloc(out, size);
-      if (e != hipSuccess && kept_ > 0) {
-        (void)hipGetLastError();
-        give_back();
-        e = hipMalloc(out, size);
-      }
-      if (e != hipSuccess) {
-        (void)hipGetLastError();
-        *out = nullptr;
-        return e;
-      }
-    }
-    owned_.emplace(*out, size);
-    return hipSuccess;
-  }
-
-  // False when this session did not allocate ptr.
-  bool free(void* ptr, hipError_t* status) {
-    *status = hipSuccess;
-    std::lock_guard<std::mutex> lock(mutex_);
-    const auto it = owned_.find(ptr);
-    if (it == owned_.end()) return false;
-    const size_t size = it->second;
-    owned_.erase(it);
-    if (size <= kMostBytes) {
-      if (kept_ + size > kKeepBytes) give_back();
-      resting_.push_back({size, ptr});
-      ++resting_classes_[size];
-      kept_ += size;
-      return true;
-    }
-    *status = hipStreamSynchronize(stream_);
-    const hipError_t e = hipFree(ptr);
-    if (*status == hipSuccess) *status = e;
-    return true;
-  }
-
-  // Everything, live allocations too (the session's work has ended).
-  void release_all() {
-    std::lock_guard<std::mutex> lock(mutex_);
-    give_back();
-    for (const auto& block : owned_) (void)hipFree(block.first);
-    owned_.clear();
-  }
-
- private:
-  static constexpr size_t kKeepBytes = size_t(1) << 30;
-  static constexpr size_t kMostBytes = size_t(256) << 20;
-  static constexpr size_t kRest = 16;
-
-  // Sizes round up to eighths of a power of two, at least 256 bytes.
-  static size_t size_class(size_t bytes) {
-    size_t unit = 256;
-    while (unit * 16 < bytes) unit *= 2;
-    return (bytes + unit - 1) / unit * unit + (bytes == 0 ? unit : 0);
-  }
-  bool capturing() const {
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    const hipError_t e = hipStreamIsCapturing(stream_, &capture);
-    if (e != hipSuccess) (void)hipGetLastError();
-    return e != hipSuccess || capture != hipStreamCaptureStatusNone;
-  }
-  // Whether a resting block of this class is worth waiting for the device:
-  // kRest of them rest (of a large class, half of what is kept), or the
-  // session's own work is done, so that there is hardly anything to wait for.
-  bool worth_a_wait(size_t size) const {
-    const auto it = resting_classes_.find(size);
-    if (it == resting_classes_.end()) return false;
-    if (it->second >= kRest || it->second * size >= kKeepBytes / 2) return true;
-    if (capturing()) return false;
-    const hipError_t e = hipStreamQuery(stream_);
-    if (e != hipSuccess) (void)hipGetLastError();
-    return e == hipSuccess;
-  }
-  // Waits for the device and makes the resting blocks ready; false (nothing
-  // changed) where it cannot wait now, as while the stream is captured.
-  bool settle() {
-    if (capturing()) return false;
-    if (hipDeviceSynchronize() != hipSuccess) {
-      (void)hipGetLastError();
-      return false;
-    }
-    for (const Block& b : resting_) ready_[b.size].push_back(b.ptr);
-    resting_.clear();
-    resting_classes_.clear();
-    return true;
-  }
-  // Returns every kept block to the runtime, which waits for its users too.
-  void give_back() {
-    if (!resting_.empty()) (void)settle();
-    for (const Block& b : resting_) (void)hipFree(b.ptr);
-    for (const auto& entry : ready_)
-      for (void* ptr : entry.second) (void)hipFree(ptr);
-    resting_.clear();
-    resting_classes_.clear();
-    ready_.clear();
-    kept_ = 0;
-  }
-
-  struct Block {
-    size_t size;
-    void* ptr;
-  };
-  hipStream_t stream_;
-  std::mutex mutex_;
-  std::unordered_map<void*, size_t> owned_;  // handed out: size class by address
-  std::map<size_t, std::vector<void*>> ready_;
-  std::vector<Block> resting_;
-  std::unordered_map<size_t, size_t> resting_classes_;
-  size_t kept_ = 0;  // bytes of ready_ and resting_
-};
 
 struct affon_rocm_session {
   int device = 0;
@@ -171,48 +26,8 @@ struct affon_rocm_session {
   affon::Workspace* workspace = nullptr;
   // Allocations made through affon_rocm_alloc; the session frees those still
   // live when it ends, so tensors that outlive it leak nothing.
-  DeviceMemory* memory = nullptr;
+  affon::DeviceMemory* memory = nullptr;
 };
-
-namespace affon {
-
-Workspace::~Workspace() {
-  if (hipSetDevice(device_) != hipSuccess) return;
-  if (ptr_ != nullptr) (void)hipFree(ptr_);
-  for (void* p : retired_) (void)hipFree(p);
-}
-
-void* Workspace::get(size_t bytes) {
-  if (bytes <= bytes_) return ptr_;
-  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(stream_, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return nullptr;
-  // The old buffer stays allocated (retired) until the session ends: work
-  // already enqueued, and graphs captured with its address, may still use it.
-  if (ptr_ != nullptr) {
-    retired_.push_back(ptr_);
-    retired_bytes_ = bytes_;
-  }
-  ptr_ = nullptr;
-  bytes_ = 0;
-  // Grow at least twofold, so that retired buffers stay few.
-  const size_t want = bytes > 2 * retired_bytes_ ? bytes : 2 * retired_bytes_;
-  const size_t rounded = (want + (size_t(1) << 20) - 1) & ~((size_t(1) << 20) - 1);
-  if (hipMalloc(&ptr_, rounded) != hipSuccess) {
-    ptr_ = nullptr;
-    (void)hipGetLastError();
-    return nullptr;
-  }
-  if (hipMemset(ptr_, 0, rounded) != hipSuccess) {
-    (void)hipFree(ptr_);
-    ptr_ = nullptr;
-    (void)hipGetLastError();
-    return nullptr;
-  }
-  bytes_ = rounded;
-  return ptr_;
-}
-
-}  // namespace affon
 
 // Scratch memory of affon_rocm_quantized_matmul_noalloc: the split-K partial
 // sums of the tiled kernels and the reassociated prefill GEMM's per-group
@@ -474,7 +289,7 @@ int affon_rocm_session_create(int device, affon_rocm_session** out) {
   session->device = device;
   session->stream = stream;
   session->workspace = new affon::Workspace(device, stream);
-  session->memory = new DeviceMemory(stream);
+  session->memory = new affon::DeviceMemory(stream);
   *out = session;
   return AFFON_ROCM_OK;
 }

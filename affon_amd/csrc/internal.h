@@ -3,10 +3,10 @@
 
 #include <hip/hip_runtime.h>
 #include <cstdint>
-#include <vector>
 
 #include "affon_rocm.h"
 #include "epilogue.h"
+#include "memory.h"
 
 namespace affon {
 
@@ -28,53 +28,6 @@ struct QmmProblem {
   int p_dtype = AFFON_ROCM_F32;
   float* out = nullptr;
   Epilogue epi;  // applied by the kernel that stores each output element
-};
-
-// Device scratch memory owned by a session and ordered by its stream.
-// Buffers it outgrows are retired, not freed, until the session ends: a
-// graph captured earlier keeps the old address in its kernel arguments and
-// may still be replayed.
-class Workspace {
- public:
-  Workspace(int device, hipStream_t stream) : device_(device), stream_(stream) {}
-  ~Workspace();
-  Workspace(const Workspace&) = delete;
-  Workspace& operator=(const Workspace&) = delete;
-  // At least `bytes` of device memory, or nullptr when it cannot grow now
-  // (the stream is being captured into a graph, or the allocation failed).
-  void* get(size_t bytes);
-  size_t retired() const { return retired_.size(); }
-
- private:
-  int device_;
-  hipStream_t stream_;
-  void* ptr_ = nullptr;
-  size_t bytes_ = 0;
-  std::vector<void*> retired_;
-  size_t retired_bytes_ = 0;  // size of the last retired buffer
-};
-
-// Where a launcher enqueues its work, and the scratch memory it may use for
-// split-K partial sums: the session's workspace (grown on demand), or a
-// fixed buffer of fixed_bytes (the no-allocation entry point), or none.
-struct Launch {
-  hipStream_t stream = nullptr;
-  Workspace* workspace = nullptr;
-  void* fixed = nullptr;
-  size_t fixed_bytes = 0;
-  // Set when a fixed buffer is too small for the launcher's plan; the
-  // launcher then launches nothing and returns hipErrorOutOfMemory.
-  mutable size_t fixed_short = 0;
-
-  bool can_split() const { return workspace != nullptr || fixed != nullptr; }
-  // At least `bytes` of scratch, or nullptr (workspace: it cannot grow now;
-  // fixed buffer: too small, recorded in fixed_short).
-  void* scratch(size_t bytes) const {
-    if (workspace != nullptr) return workspace->get(bytes);
-    if (fixed != nullptr && bytes <= fixed_bytes) return fixed;
-    if (fixed != nullptr) fixed_short = bytes;
-    return nullptr;
-  }
 };
 
 // Per-candidate capability guards and launchers. A guard returns true when
