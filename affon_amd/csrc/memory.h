@@ -71,6 +71,12 @@ struct Launch {
 // goes back to the runtime, as everything does when an allocation fails and
 // when the session ends.
 //
+// A graph holds the addresses that its captured region used, and writes to
+// them in every replay. What is allocated or freed while the session's stream
+// is captured is therefore never handed out again, and is released when the
+// session ends (as Workspace does with buffers it outgrew). While a capture
+// lasts nothing goes back to the runtime.
+//
 // alloc and free may come from any thread (a caller's garbage collector
 // frees from whichever thread it runs on): the mutex guards everything.
 class DeviceMemory {
@@ -100,7 +106,7 @@ class DeviceMemory {
         return e;
       }
     }
-    owned_.emplace(*out, size);
+    owned_.emplace(*out, Owned{size, capturing()});
     return hipSuccess;
   }
 
@@ -110,14 +116,21 @@ class DeviceMemory {
     std::lock_guard<std::mutex> lock(mutex_);
     const auto it = owned_.find(ptr);
     if (it == owned_.end()) return false;
-    const size_t size = it->second;
+    const size_t size = it->second.size;
+    if (it->second.captured || capturing()) {
+      retired_.push_back(ptr);
+      owned_.erase(it);
+      return true;
+    }
     owned_.erase(it);
     if (size <= kMostBytes) {
       if (kept_ + size > kKeepBytes) give_back();
-      resting_.push_back({size, ptr});
-      ++resting_classes_[size];
-      kept_ += size;
-      return true;
+      if (kept_ + size <= kKeepBytes) {
+        resting_.push_back({size, ptr});
+        ++resting_classes_[size];
+        kept_ += size;
+        return true;
+      }
     }
     *status = hipStreamSynchronize(stream_);
     const hipError_t e = hipFree(ptr);
@@ -128,9 +141,14 @@ class DeviceMemory {
   // Everything, live allocations too (the session's work has ended).
   void release_all() {
     std::lock_guard<std::mutex> lock(mutex_);
-    give_back();
+    free_all(resting_);
+    for (auto& entry : ready_) free_all(entry.second);
+    free_all(retired_);
     for (const auto& block : owned_) (void)hipFree(block.first);
+    resting_classes_.clear();
+    ready_.clear();
     owned_.clear();
+    kept_ = 0;
   }
 
  private:
@@ -175,14 +193,11 @@ class DeviceMemory {
     resting_classes_.clear();
     return true;
   }
-  // Returns every kept block to the runtime, which waits for its users too.
+  // Returns every kept block to the runtime; none where the device cannot be
+  // waited for now.
   void give_back() {
-    if (!resting_.empty()) (void)settle();
-    for (const Block& b : resting_) (void)hipFree(b.ptr);
-    for (const auto& entry : ready_)
-      for (void* ptr : entry.second) (void)hipFree(ptr);
-    resting_.clear();
-    resting_classes_.clear();
+    if (capturing() || (!resting_.empty() && !settle())) return;
+    for (auto& entry : ready_) free_all(entry.second);
     ready_.clear();
     kept_ = 0;
   }
@@ -191,11 +206,23 @@ class DeviceMemory {
     size_t size;
     void* ptr;
   };
+  struct Owned {
+    size_t size;
+    bool captured;  // allocated while the stream was captured
+  };
+  static void* address(const Block& b) { return b.ptr; }
+  static void* address(void* ptr) { return ptr; }
+  template <typename T>
+  static void free_all(std::vector<T>& blocks) {
+    for (const T& b : blocks) (void)hipFree(address(b));
+    blocks.clear();
+  }
   hipStream_t stream_;
   std::mutex mutex_;
-  std::unordered_map<void*, size_t> owned_;  // handed out: size class by address
+  std::unordered_map<void*, Owned> owned_;  // handed out, by address
   std::map<size_t, std::vector<void*>> ready_;
   std::vector<Block> resting_;
+  std::vector<void*> retired_;  // freed, but of a captured region
   std::unordered_map<size_t, size_t> resting_classes_;
   size_t kept_ = 0;  // bytes of ready_ and resting_
 };

@@ -105,8 +105,11 @@ void* affon_rocm_session_stream(affon_rocm_session* session);
 /* Device memory of the session. Freed memory is kept for later allocations of
  * the session (at most 1 GiB, no block over 256 MiB) and handed out again only
  * after the device has been idle since its free, as a return to the runtime
- * would wait for; a free does not wait. It goes back to the runtime when an
- * allocation fails for want of it and when the session ends. */
+ * would wait for; the free itself waits only where a block is not kept. It
+ * goes back to the runtime when an allocation fails for want of it and when
+ * the session ends. Memory allocated or freed while the session's stream is
+ * captured stays aside until the session ends: replays of the graph still
+ * write to it. */
 int affon_rocm_alloc(affon_rocm_session* session, size_t bytes, void** out);
 int affon_rocm_free(affon_rocm_session* session, void* ptr);
 /* Copies are ordered on the session stream and complete before returning. */

@@ -1,0 +1,118 @@
+// DeviceMemory against a stand-in HIP runtime. Run with the name of one check.
+#include <cstdio>
+#include <set>
+
+#include "memory.h"
+
+namespace {
+
+constexpr size_t MiB = size_t(1) << 20;
+
+#define CHECK(x)                                                   \
+  do {                                                             \
+    if (!(x)) {                                                    \
+      std::printf("%s:%d: %s\n", __FILE__, __LINE__, #x);          \
+      std::exit(1);                                                \
+    }                                                              \
+  } while (0)
+
+void* alloc(affon::DeviceMemory& m, size_t bytes) {
+  void* p = nullptr;
+  CHECK(m.alloc(bytes, &p) == hipSuccess && p != nullptr);
+  CHECK(fake::blocks.at(p) >= bytes);
+  return p;
+}
+void free(affon::DeviceMemory& m, void* p) {
+  hipError_t e;
+  CHECK(m.free(p, &e) && e == hipSuccess);
+}
+// Idle, what the session keeps is handed out: whether any of `ptrs` is, among many allocations.
+bool comes_back(affon::DeviceMemory& m, const std::set<void*>& ptrs, size_t bytes) {
+  for (int i = 0; i < 100; ++i)
+    if (ptrs.count(alloc(m, bytes))) return true;
+  return false;
+}
+
+void reuse() {
+  affon::DeviceMemory m(nullptr);
+  void* a = alloc(m, 5000);
+  free(m, a);
+  CHECK(alloc(m, 5000) == a);
+}
+
+// A block freed while any stream works waits for the device to be idle.
+void other_stream() {
+  affon::DeviceMemory m(nullptr);
+  void* a = alloc(m, 5000);
+  fake::session_busy = fake::device_busy = true;
+  free(m, a);
+  CHECK(alloc(m, 5000) != a && fake::device_busy);  // the session works: no wait for one block
+  fake::session_busy = false;  // only another stream works now
+  CHECK(alloc(m, 5000) == a && !fake::device_busy);
+}
+
+// What a captured region allocates or frees stays aside until the session ends.
+void capture(size_t bytes) {
+  affon::DeviceMemory m(nullptr);
+  void* before = alloc(m, bytes);
+  void* kept = alloc(m, bytes);
+  free(m, kept);
+  fake::session_capturing = true;
+  void *in = alloc(m, bytes), *out = alloc(m, bytes);
+  free(m, in);      // as a captured Program's intermediate
+  free(m, before);  // of before, used in the region
+  CHECK(alloc(m, bytes) != in);
+  CHECK(fake::frees_while_capturing == 0);
+  fake::session_capturing = false;
+  free(m, out);  // a captured output dropped later
+  if (bytes <= 256 * MiB) CHECK(!comes_back(m, {in, out, before}, bytes));
+  CHECK(fake::blocks.count(in) && fake::blocks.count(out) && fake::blocks.count(before));
+  hipError_t e;
+  CHECK(!m.free(in, &e));  // freed once
+  m.release_all();
+  CHECK(fake::blocks.empty());
+}
+
+// Nothing goes back to the runtime while the stream is captured, full pool or failing allocation.
+void no_free_in_capture() {
+  affon::DeviceMemory m(nullptr);
+  std::set<void*> parked;
+  for (int i = 0; i < 8; ++i) parked.insert(alloc(m, 100 * MiB));
+  fake::session_busy = true;
+  for (void* p : parked) free(m, p);
+  fake::session_capturing = true;
+  std::set<void*> live;
+  for (int i = 0; i < 5; ++i) live.insert(alloc(m, 100 * MiB));
+  for (void* p : live) free(m, p);
+  fake::limit = fake::used;
+  void* p = nullptr;
+  CHECK(m.alloc(64 * MiB, &p) == hipErrorOutOfMemory && p == nullptr);
+  CHECK(fake::frees_while_capturing == 0);
+  fake::session_capturing = false;
+  alloc(m, 64 * MiB);  // from what the parked blocks gave back
+}
+
+// The device cannot be waited for (another stream is captured): kept blocks stay, within the bound.
+void no_idle_moment() {
+  affon::DeviceMemory m(nullptr);
+  std::set<void*> ptrs;
+  for (int i = 0; i < 20; ++i) ptrs.insert(alloc(m, 100 * MiB));
+  fake::sync_fails = true;
+  for (void* p : ptrs) free(m, p);
+  CHECK(fake::used <= 1024 * MiB);
+  for (int i = 0; i < 20; ++i) CHECK(!ptrs.count(alloc(m, 100 * MiB)));
+}
+
+}  // namespace
+
+int main(int, char** argv) {
+  const std::string name = argv[1];
+  if (name == "reuse") reuse();
+  else if (name == "other_stream") other_stream();
+  else if (name == "capture") capture(5000);
+  else if (name == "capture_large") capture(300 * MiB);
+  else if (name == "no_free_in_capture") no_free_in_capture();
+  else if (name == "no_idle_moment") no_idle_moment();
+  else return 2;
+  return 0;
+}

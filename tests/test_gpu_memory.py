@@ -8,8 +8,10 @@ import numpy as np
 import pytest
 
 import affon_amd as A
-from affon_amd import _native
+from affon_amd import _native, ops
+from affon_amd.decoder import QuantizedDecoderBlock
 from tests.helpers import HipRuntime
+from tests.test_gpu_decoder import BITS, GROUP, SHAPE, block_checkpoint
 
 pytestmark = pytest.mark.gpu
 MIB = 1 << 20
@@ -91,3 +93,60 @@ def test_frees_from_other_threads(session):
         dropped.clear()
         gc.collect()
     assert not errors
+
+
+def test_memory_of_a_captured_program_stays_its_own(tmp_path, rng):
+    """A captured feed-forward frees its gated product inside the region, and
+    its output is dropped after it. Every replay writes to both: tensors made
+    since then keep their values."""
+    hip, rows = HipRuntime(), 32
+    path, _ = block_checkpoint(tmp_path)
+    with A.Session("rocm") as session:
+        block = QuantizedDecoderBlock.from_checkpoint(session, path, 3, SHAPE, bits=BITS, group_size=GROUP)
+        x = session.from_bytes(A.core.bf16_bits(rng.standard_normal((rows, SHAPE.width)).astype(np.float32)),
+                               A.TensorSpec.bf16((rows, SHAPE.width)))
+        want = block.feed_forward(x).numpy()
+        for _ in range(3):
+            block.feed_forward(x)
+            session.synchronize()
+        # Blocks of both sizes are ready to be handed out within the region.
+        for width in (SHAPE.inner_width, SHAPE.width):
+            session.empty("f32", (rows, width))
+        kept = []
+        graph = hip.capture(session.stream, lambda: kept.append(block.feed_forward(x)))
+        try:
+            hip.replay(session.stream, graph)
+            np.testing.assert_array_equal(kept[0].numpy(), want)
+            kept.clear()
+            session.synchronize()
+            tensors = [session.tensor(np.full((rows, width), i, np.float32))
+                       for i in range(24) for width in (SHAPE.inner_width, SHAPE.width)]
+            for _ in range(3):
+                hip.replay(session.stream, graph)
+                block.feed_forward(x)
+                for i, t in enumerate(tensors):
+                    assert (t.numpy() == i // 2).all(), i
+        finally:
+            hip.destroy(graph)
+
+
+def test_memory_used_on_another_stream(rng):
+    """A block freed while another session's stream still writes to it is
+    handed out only after that work has ended."""
+    M, N, K = 512, 4096, 4096
+    with A.Session("rocm") as one, A.Session("rocm") as other:
+        x = other.tensor(rng.standard_normal((M, K)).astype(np.float32))
+        w = A.quantize(other.tensor(rng.standard_normal((N, K)).astype(np.float32)), bits=4, group_size=64,
+                       param_dtype="f32")
+        A.quantized_matmul(x, *w, bits=4, group_size=64)
+        other.synchronize()
+        block = raw_alloc(one, M * N * 4)
+        desc = ops._descriptor(x, *w, 4, 64, None, "auto", "backend_equivalent")
+        desc.output, desc.output_bytes = block, M * N * 4
+        for _ in range(100):  # some milliseconds
+            assert _native.load().affon_rocm_quantized_matmul(other._handle, ctypes.byref(desc)) == 0
+        assert _native.load().affon_rocm_free(one._handle, block) == 0
+        tensors = [one.tensor(np.full((M, N), i, np.float32)) for i in range(3)]
+        other.synchronize()
+        for i, t in enumerate(tensors):
+            assert (t.numpy() == i).all()
