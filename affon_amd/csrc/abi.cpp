@@ -13,6 +13,7 @@
 #include <cstring>
 #include <exception>
 #include <limits>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -285,12 +286,16 @@ int affon_rocm_session_create(int device, affon_rocm_session** out) {
   if ((e = hipSetDevice(device)) != hipSuccess) return hip_fail(e, "hipSetDevice");
   hipStream_t stream = nullptr;
   if ((e = hipStreamCreateWithFlags(&stream, hipStreamNonBlocking)) != hipSuccess) return hip_fail(e, "hipStreamCreate");
-  auto* session = new affon_rocm_session;
-  session->device = device;
-  session->stream = stream;
-  session->workspace = new affon::Workspace(device, stream);
-  session->memory = new affon::DeviceMemory(stream);
-  *out = session;
+  try {
+    auto workspace = std::make_unique<affon::Workspace>(device, stream);
+    auto memory = std::make_unique<affon::DeviceMemory>(stream);
+    *out = new affon_rocm_session{device, stream, workspace.get(), memory.get()};
+    workspace.release();
+    memory.release();
+  } catch (const std::exception& error) {
+    (void)hipStreamDestroy(stream);
+    return fail(AFFON_ROCM_CORE_FAILURE, "session_create: %s", error.what());
+  }
   return AFFON_ROCM_OK;
 }
 

@@ -78,7 +78,8 @@ struct Launch {
 // lasts nothing goes back to the runtime.
 //
 // alloc and free may come from any thread (a caller's garbage collector
-// frees from whichever thread it runs on): the mutex guards everything.
+// frees from whichever thread it runs on): the mutex guards everything. Both
+// may throw std::bad_alloc; a block is then where it was, or (alloc) returned.
 class DeviceMemory {
  public:
   explicit DeviceMemory(hipStream_t stream) : stream_(stream) {}
@@ -86,12 +87,11 @@ class DeviceMemory {
   hipError_t alloc(size_t bytes, void** out) {
     const size_t size = bytes <= kMostBytes ? size_class(bytes) : bytes;
     std::lock_guard<std::mutex> lock(mutex_);
-    auto ready = ready_.find(size);
-    if (ready == ready_.end() && worth_a_wait(size) && settle()) ready = ready_.find(size);
-    if (ready != ready_.end()) {
-      *out = ready->second.back();
-      ready->second.pop_back();
-      if (ready->second.empty()) ready_.erase(ready);
+    std::vector<void*>* ready = find_ready(size);
+    if (ready == nullptr && worth_a_wait(size) && settle()) ready = find_ready(size);
+    if (ready != nullptr) {
+      *out = ready->back();
+      ready->pop_back();
       kept_ -= size;
     } else {
       hipError_t e = hipMalloc(out, size);
@@ -106,7 +106,13 @@ class DeviceMemory {
         return e;
       }
     }
-    owned_.emplace(*out, Owned{size, capturing()});
+    try {
+      owned_.emplace(*out, Owned{size, capturing()});
+    } catch (...) {
+      (void)hipFree(*out);
+      *out = nullptr;
+      throw;
+    }
     return hipSuccess;
   }
 
@@ -122,16 +128,18 @@ class DeviceMemory {
       owned_.erase(it);
       return true;
     }
-    owned_.erase(it);
     if (size <= kMostBytes) {
       if (kept_ + size > kKeepBytes) give_back();
       if (kept_ + size <= kKeepBytes) {
+        size_t& resting = resting_classes_[size];
         resting_.push_back({size, ptr});
-        ++resting_classes_[size];
+        ++resting;
         kept_ += size;
+        owned_.erase(it);
         return true;
       }
     }
+    owned_.erase(it);
     *status = hipStreamSynchronize(stream_);
     const hipError_t e = hipFree(ptr);
     if (*status == hipSuccess) *status = e;
@@ -162,6 +170,11 @@ class DeviceMemory {
     while (unit * 16 < bytes) unit *= 2;
     return (bytes + unit - 1) / unit * unit + (bytes == 0 ? unit : 0);
   }
+  // The blocks of this class that can be handed out, if there are any.
+  std::vector<void*>* find_ready(size_t size) {
+    const auto it = ready_.find(size);
+    return it == ready_.end() || it->second.empty() ? nullptr : &it->second;
+  }
   bool capturing() const {
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     const hipError_t e = hipStreamIsCapturing(stream_, &capture);
@@ -188,8 +201,12 @@ class DeviceMemory {
       (void)hipGetLastError();
       return false;
     }
-    for (const Block& b : resting_) ready_[b.size].push_back(b.ptr);
-    resting_.clear();
+    while (!resting_.empty()) {  // a block at a time: it is in one list, whatever throws
+      const Block b = resting_.back();
+      ready_[b.size].push_back(b.ptr);
+      resting_.pop_back();
+      --resting_classes_[b.size];
+    }
     resting_classes_.clear();
     return true;
   }

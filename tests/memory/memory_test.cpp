@@ -1,10 +1,14 @@
 // DeviceMemory against a stand-in HIP runtime. Run with the name of one check.
 #include <cstdio>
+#include <new>
 #include <set>
 
 #include "memory.h"
 
 namespace {
+
+// Allocations on the host until one fails (-1: none does).
+int g_until_bad_alloc = -1;
 
 constexpr size_t MiB = size_t(1) << 20;
 
@@ -103,7 +107,45 @@ void no_idle_moment() {
   for (int i = 0; i < 20; ++i) CHECK(!ptrs.count(alloc(m, 100 * MiB)));
 }
 
+// Whichever allocation on the host fails, no block is lost, given twice or freed twice.
+void host_memory_fails() {
+  for (int n = 0; n < 60; ++n) {
+    affon::DeviceMemory m(nullptr);
+    std::set<void*> live;
+    g_until_bad_alloc = n;
+    for (int i = 0; i < 200; ++i) {
+      try {
+        if (i % 40 < 20) {
+          void* p = nullptr;
+          if (m.alloc(1000 + 300 * (i % 3), &p) == hipSuccess) {
+            const int armed = g_until_bad_alloc;
+            g_until_bad_alloc = -1;
+            CHECK(live.insert(p).second && fake::blocks.count(p));
+            g_until_bad_alloc = armed;
+          }
+        } else if (!live.empty()) {
+          hipError_t e;
+          void* p = *live.begin();
+          CHECK(m.free(p, &e));
+          live.erase(p);
+        }
+      } catch (const std::bad_alloc&) {
+      }
+    }
+    g_until_bad_alloc = -1;
+    m.release_all();
+    CHECK(fake::blocks.empty());
+  }
+}
+
 }  // namespace
+
+void* operator new(size_t bytes) {
+  if (g_until_bad_alloc >= 0 && g_until_bad_alloc-- == 0) throw std::bad_alloc();
+  return std::malloc(bytes);
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
 
 int main(int, char** argv) {
   const std::string name = argv[1];
@@ -113,6 +155,7 @@ int main(int, char** argv) {
   else if (name == "capture_large") capture(300 * MiB);
   else if (name == "no_free_in_capture") no_free_in_capture();
   else if (name == "no_idle_moment") no_idle_moment();
+  else if (name == "host_memory_fails") host_memory_fails();
   else return 2;
   return 0;
 }
