@@ -85,7 +85,8 @@ class DeviceMemory {
   explicit DeviceMemory(hipStream_t stream) : stream_(stream) {}
 
   hipError_t alloc(size_t bytes, void** out) {
-    const size_t size = bytes <= kMostBytes ? size_class(bytes) : bytes;
+    size_t size = bytes <= kMostBytes ? size_class(bytes) : bytes;
+    bool pooled = size <= kMostBytes;
     std::lock_guard<std::mutex> lock(mutex_);
     std::vector<void*>* ready = find_ready(size);
     if (ready == nullptr && worth_a_wait(size) && settle()) ready = find_ready(size);
@@ -100,6 +101,12 @@ class DeviceMemory {
         give_back();
         e = hipMalloc(out, size);
       }
+      if (e != hipSuccess && size > bytes && bytes > 0) {  // what the rounding up asks for may be too much
+        (void)hipGetLastError();
+        size = bytes;
+        pooled = false;
+        e = hipMalloc(out, size);
+      }
       if (e != hipSuccess) {
         (void)hipGetLastError();
         *out = nullptr;
@@ -107,7 +114,7 @@ class DeviceMemory {
       }
     }
     try {
-      owned_.emplace(*out, Owned{size, capturing()});
+      owned_.emplace(*out, Owned{size, pooled, capturing()});
     } catch (...) {
       (void)hipFree(*out);
       *out = nullptr;
@@ -128,7 +135,7 @@ class DeviceMemory {
       owned_.erase(it);
       return true;
     }
-    if (size <= kMostBytes) {
+    if (it->second.pooled) {
       if (kept_ + size > kKeepBytes) give_back();
       if (kept_ + size <= kKeepBytes) {
         size_t& resting = resting_classes_[size];
@@ -225,6 +232,7 @@ class DeviceMemory {
   };
   struct Owned {
     size_t size;
+    bool pooled;    // of a size class, kept when freed
     bool captured;  // allocated while the stream was captured
   };
   static void* address(const Block& b) { return b.ptr; }

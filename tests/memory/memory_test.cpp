@@ -107,6 +107,16 @@ void no_idle_moment() {
   for (int i = 0; i < 20; ++i) CHECK(!ptrs.count(alloc(m, 100 * MiB)));
 }
 
+// A size that fits only without rounding up is still given.
+void exact_size() {
+  affon::DeviceMemory m(nullptr);
+  fake::limit = 17 * MiB + 4096;
+  void* p = alloc(m, 17 * MiB + 1);
+  free(m, p);
+  CHECK(fake::used == 0);
+  alloc(m, 17 * MiB + 2);
+}
+
 // Whichever allocation on the host fails, no block is lost, given twice or freed twice.
 void host_memory_fails() {
   for (int n = 0; n < 60; ++n) {
@@ -155,6 +165,7 @@ int main(int, char** argv) {
   else if (name == "capture_large") capture(300 * MiB);
   else if (name == "no_free_in_capture") no_free_in_capture();
   else if (name == "no_idle_moment") no_idle_moment();
+  else if (name == "exact_size") exact_size();
   else if (name == "host_memory_fails") host_memory_fails();
   else return 2;
   return 0;
