@@ -24,8 +24,10 @@ class Workspace {
   // (the stream is being captured into a graph, or the allocation failed).
   void* get(size_t bytes);
   size_t retired() const { return retired_.size(); }
+  std::mutex& mutex() { return mutex_; }
 
  private:
+  std::mutex mutex_;
   int device_;
   hipStream_t stream_;
   void* ptr_ = nullptr;
@@ -37,6 +39,10 @@ class Workspace {
 // Where a launcher enqueues its work, and the scratch memory it may use for
 // split-K partial sums: the session's workspace (grown on demand), or a
 // fixed buffer of fixed_bytes (the no-allocation entry point), or none.
+//
+// A call that takes the workspace holds it until the call ends, so that the
+// launches that fill and read it are enqueued with no other thread's between
+// them; on the stream they then run in that order.
 struct Launch {
   hipStream_t stream = nullptr;
   Workspace* workspace = nullptr;
@@ -45,12 +51,16 @@ struct Launch {
   // Set when a fixed buffer is too small for the launcher's plan; the
   // launcher then launches nothing and returns hipErrorOutOfMemory.
   mutable size_t fixed_short = 0;
+  mutable std::unique_lock<std::mutex> held;
 
   bool can_split() const { return workspace != nullptr || fixed != nullptr; }
   // At least `bytes` of scratch, or nullptr (workspace: it cannot grow now;
   // fixed buffer: too small, recorded in fixed_short).
   void* scratch(size_t bytes) const {
-    if (workspace != nullptr) return workspace->get(bytes);
+    if (workspace != nullptr) {
+      if (!held.owns_lock()) held = std::unique_lock<std::mutex>(workspace->mutex());
+      return workspace->get(bytes);
+    }
     if (fixed != nullptr && bytes <= fixed_bytes) return fixed;
     if (fixed != nullptr) fixed_short = bytes;
     return nullptr;

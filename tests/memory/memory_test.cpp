@@ -1,7 +1,10 @@
-// DeviceMemory against a stand-in HIP runtime. Run with the name of one check.
+// DeviceMemory and Workspace against a stand-in HIP runtime. Run with the name of one check.
+#include <atomic>
+#include <chrono>
 #include <cstdio>
 #include <new>
 #include <set>
+#include <thread>
 
 #include "memory.h"
 
@@ -148,6 +151,28 @@ void host_memory_fails() {
   }
 }
 
+// A call's scratch is its own until the call ends, whichever threads call.
+void scratch_between_threads() {
+  affon::Workspace workspace(0, nullptr);
+  std::atomic<bool> taken{false}, ended{false};
+  std::thread first([&] {
+    {
+      affon::Launch l;
+      l.workspace = &workspace;
+      CHECK(l.scratch(1000) != nullptr && l.scratch(2000) != nullptr);  // taken twice by one call
+      taken = true;
+      std::this_thread::sleep_for(std::chrono::milliseconds(200));
+      ended = true;
+    }
+  });
+  while (!taken) std::this_thread::yield();
+  affon::Launch l;
+  l.workspace = &workspace;
+  CHECK(l.scratch(1000) != nullptr);
+  CHECK(ended);
+  first.join();
+}
+
 }  // namespace
 
 void* operator new(size_t bytes) {
@@ -166,6 +191,7 @@ int main(int, char** argv) {
   else if (name == "no_free_in_capture") no_free_in_capture();
   else if (name == "no_idle_moment") no_idle_moment();
   else if (name == "exact_size") exact_size();
+  else if (name == "scratch_between_threads") scratch_between_threads();
   else if (name == "host_memory_fails") host_memory_fails();
   else return 2;
   return 0;

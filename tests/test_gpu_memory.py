@@ -150,3 +150,39 @@ def test_memory_used_on_another_stream(rng):
         other.synchronize()
         for i, t in enumerate(tensors):
             assert (t.numpy() == i).all()
+
+
+def test_scratch_between_threads(session, rng):
+    """Calls that keep partial results in the session's scratch memory between
+    two launches (softmax of few long rows, a batch in K ranges), from two
+    threads at once: each gets the result that it gets alone."""
+    errors = []
+
+    def softmax(seed):
+        x = session.tensor(np.random.default_rng(seed).standard_normal((3, 40000)).astype(np.float32))
+        return lambda: A.softmax(x, -1).numpy()
+
+    def batch(seed):
+        r = np.random.default_rng(seed)
+        x = session.tensor(r.standard_normal((40, 4096)).astype(np.float32))
+        w = A.quantize(session.tensor(r.standard_normal((512, 4096)).astype(np.float32)), bits=4, group_size=64,
+                       param_dtype="f32")
+        return lambda: A.quantized_matmul(x, *w, bits=4, group_size=64).numpy()
+
+    calls = [softmax(1), batch(2), softmax(3), batch(4)]
+    alone = [call() for call in calls]
+
+    def work(mine):
+        try:
+            for _ in range(100):
+                for i in mine:
+                    np.testing.assert_array_equal(calls[i](), alone[i])
+        except Exception as e:  # noqa: BLE001 - reported below
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(mine,)) for mine in ((0, 1), (2, 3))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors[0]
