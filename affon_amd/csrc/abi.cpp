@@ -907,8 +907,14 @@ struct DeviceBuffer {
   affon_rocm_session* session;
   void* ptr = nullptr;
   explicit DeviceBuffer(affon_rocm_session* s) : session(s) {}
+  // Not affon_rocm_free, which clears the message of the step that failed.
   ~DeviceBuffer() {
-    if (ptr != nullptr) (void)affon_rocm_free(session, ptr);
+    if (ptr == nullptr) return;
+    try {
+      hipError_t e = hipSetDevice(session->device);
+      (void)session->memory->free(ptr, &e);
+    } catch (const std::exception&) {  // the block then goes when the session ends
+    }
   }
 };
 

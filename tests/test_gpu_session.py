@@ -1,6 +1,8 @@
 """Session resource rules on the GPU: scratch memory that a captured graph
 still uses survives the session's later growth, and disposing a Session
 frees the device memory of tensors that are still alive."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -73,3 +75,18 @@ def test_dispose_frees_live_tensors():
     with pytest.raises(RuntimeError, match="disposed"):
         held[0].numpy()
     del held  # releasing after dispose frees nothing twice
+
+
+def test_host_entry_reports_a_late_failure():
+    """The host-pointer entry point fails after some of its buffers are there
+    (its output, 4 TiB, does not fit any device): the message says so."""
+    rows, depth, columns = 1 << 20, 16, 1 << 20
+    x = np.zeros(rows * depth, np.float32)
+    w, s = np.zeros(columns, np.uint32), np.zeros(columns, np.float32)
+    out = np.zeros(1, np.float32)  # not reached
+    lib = _native.load()
+    p = lambda a: ctypes.c_void_p(a.ctypes.data)
+    status = lib.compute_core_run_quantized_matmul_f32(p(x), x.size, p(w), w.size, p(s), s.size, p(s), s.size, p(out),
+                                                       rows * columns, rows, depth, columns, 2, 16)
+    assert status == _native.CORE_FAILURE
+    assert "memory" in _native.last_error().lower(), _native.last_error()
