@@ -88,3 +88,38 @@ def test_index_select_rows_in_pieces(session, dtype, rng):
         want = np.where(((index >= 0) & (index < 9))[:, None], x[np.clip(index, 0, 8)], 0)
         got = A.index_select(upload(session, x, dtype), 0, session.tensor(index, "i64")).storage()
         np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_short_rows_at_the_edges_of_their_shapes(session, dtype, rng):
+    """Rows of a value per lane, rows that share a wave and rows that a wave or
+    a workgroup holds: columns on both sides of every line between them and
+    with a part of a vector at the end, rows around the line between few and
+    many and around the waves and workgroups that rows share."""
+    w = 4 if dtype == "f32" else 8  # values of a vector
+    short = [1, 2, w + 1, 4 * w, 4 * w + 1, 8 * w, 8 * w + 3, 64, 65, 16 * w, 16 * w + 1, 128, 129, 32 * w, 32 * w + 1,
+             40 * w, 40 * w + 1]
+    long = [64 * w, 64 * w + 1, 128 * w, 128 * w + 3, 256 * w, 256 * w + 1, 512 * w, 512 * w + 1, 1024 * w, 1024 * w + 1]
+    for rows, widths in ((3, short + long), (8192, short), (8193, short), (8209, short[-4:] + long[:2]), (67, long)):
+        for cols in widths:
+            x = storage(rng.standard_normal((rows, cols)) * 3, dtype)
+            x[rows // 2, cols // 2] = storage([-np.inf], dtype)[0] if cols > 1 else x[rows // 2, 0]
+            t, v = upload(session, x, dtype), widened(x)
+            check(A.softmax(t, -1).storage(), softmax_f64(v), dtype)
+            x[rows // 2, cols // 2] = 0
+            t, v = upload(session, x, dtype), widened(x)
+            check(A.rms_norm(t, -1).storage(), v / np.sqrt((v * v).mean(1, keepdims=True) + 1e-5), dtype)
+
+
+@pytest.mark.parametrize("rows,cols", [(6, 20), (6, 100), (6, 200), (8196, 20), (8196, 70), (6, 1000), (6, 3000)])
+def test_short_softmax_of_masks_and_specials(session, rows, cols, rng):
+    """As for long rows: masked values give zeros, a NaN, a +inf or -inf alone a
+    row of NaNs, and no row touches its neighbours."""
+    x = rng.standard_normal((rows, cols)).astype(np.float32)
+    x[0, cols // 3:] = -np.inf
+    x[1, : cols - 1] = np.finfo(np.float32).min
+    x[2] = -np.inf
+    x[3, cols // 2] = np.nan
+    x[4, cols - 1] = np.inf
+    x[5] = np.finfo(np.float32).min
+    check(A.softmax(upload(session, x, "f32"), -1).storage(), softmax_f64(x.astype(np.float64)), "f32")
