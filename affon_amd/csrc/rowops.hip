@@ -14,8 +14,9 @@
 // hold it in a few loads each, up to a workgroup, against one wave per row with
 // one element per lane and load before. Device us, before -> now: softmax f32
 // 32 x 128256 944 -> 12, 512 x 128256 2485 -> 145 (3.6 TB/s), 512 x 4096 33 ->
-// 4.5; rms_norm f32 32 x 4096 19 -> 2.8, bf16 512 x 4096 22 -> 4.1. The sums of many short partial sums are also nearer: softmax
-// over 128256 values 3.3e-6 -> 7.5e-8 off 64 bits.
+// 4.5; rms_norm f32 32 x 4096 19 -> 2.8, bf16 512 x 4096 22 -> 4.1. The sums
+// of many short partial sums are also nearer: softmax over 128256 values 3.3e-6
+// -> 7.5e-8 off 64 bits.
 
 #include <algorithm>
 #include <type_traits>
@@ -318,18 +319,30 @@ __global__ __launch_bounds__(256) void softmax_write_kernel(const uint8_t* x, ui
 }
 
 // out[i, :] = x[index[i], :]: raw copies of U-sized pieces, `pieces` to a row,
-// workgroups of 256 pieces of one row (grid y strides over the rows).
+// 256 consecutive ones of the output per workgroup, whichever rows they are of
+// (one division for the workgroup's first row; where it is of one or two rows,
+// a comparison finds a thread's). Workgroups of one row idle past its end: f32,
+// device us, 1000000 rows of 4 148 against 5.3, 20000 of 257 20 and 14, 20000
+// of 1024 24 and 25; a thread per element of 4 bytes 8.4, 14 and 44.
 template <typename U>
 __global__ __launch_bounds__(256) void select_rows_kernel(const U* x, U* out, int64_t rows, int64_t pieces,
                                                           const int64_t* index, int64_t count) {
-  const int64_t p = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (p >= pieces) return;
-  for (int64_t i = blockIdx.y; i < count; i += gridDim.y) {
-    const int64_t sel = index[i];
-    U v{};
-    if (sel >= 0 && sel < rows) v = x[sel * pieces + p];
-    out[i * pieces + p] = v;
+  const int64_t first = static_cast<int64_t>(blockIdx.x) * 256;
+  int64_t i = first / pieces;
+  int64_t p = first - i * pieces + threadIdx.x;
+  if (pieces < 256) {
+    const uint32_t at = static_cast<uint32_t>(p), n = static_cast<uint32_t>(pieces);
+    i += at / n;
+    p = at % n;
+  } else if (p >= pieces) {
+    ++i;
+    p -= pieces;
   }
+  if (i >= count) return;
+  const int64_t sel = index[i];
+  U v{};
+  if (sel >= 0 && sel < rows) v = x[sel * pieces + p];
+  out[first + threadIdx.x] = v;
 }
 
 // out[r, i] = x[r, index[i]], one thread per output element.
@@ -462,9 +475,8 @@ template <typename U>
 hipError_t select_rows(const void* x, int64_t rows, int64_t row_bytes, const int64_t* index, int64_t count, void* out,
                        hipStream_t stream) {
   const int64_t pieces = row_bytes / static_cast<int64_t>(sizeof(U));
-  const dim3 grid(static_cast<unsigned>((pieces + 255) / 256), static_cast<unsigned>(std::min<int64_t>(count, 32768)));
-  hipLaunchKernelGGL(select_rows_kernel<U>, grid, dim3(256), 0, stream, static_cast<const U*>(x), static_cast<U*>(out),
-                     rows, pieces, index, count);
+  hipLaunchKernelGGL(select_rows_kernel<U>, dim3(static_cast<unsigned>((count * pieces + 255) / 256)), dim3(256), 0, stream,
+                     static_cast<const U*>(x), static_cast<U*>(out), rows, pieces, index, count);
   return hipGetLastError();
 }
 }  // namespace
@@ -473,12 +485,12 @@ hipError_t index_select_launch(const void* x, int dtype, int64_t rows, int64_t c
                                int64_t count, void* out, hipStream_t stream) {
   const bool half = dtype == AFFON_ROCM_BF16;
   if (axis == 0) {
-    // Rows in 16-byte pieces where every row starts at one, else by element.
+    // Rows in the largest pieces of 16, 4 or 2 bytes that every row starts at.
     const int64_t row_bytes = cols * (half ? 2 : 4);
-    if (row_bytes % 16 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0)
-      return select_rows<u32x4_t>(x, rows, row_bytes, index, count, out, stream);
-    return half ? select_rows<uint16_t>(x, rows, row_bytes, index, count, out, stream)
-                : select_rows<uint32_t>(x, rows, row_bytes, index, count, out, stream);
+    const uint64_t starts = static_cast<uint64_t>(row_bytes) | reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out);
+    if (starts % 16 == 0) return select_rows<u32x4_t>(x, rows, row_bytes, index, count, out, stream);
+    if (starts % 4 == 0) return select_rows<uint32_t>(x, rows, row_bytes, index, count, out, stream);
+    return select_rows<uint16_t>(x, rows, row_bytes, index, count, out, stream);
   }
   const dim3 grid(static_cast<unsigned>((rows * count + 255) / 256));
   const auto* xi = static_cast<const uint8_t*>(x);

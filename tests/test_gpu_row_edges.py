@@ -123,3 +123,15 @@ def test_short_softmax_of_masks_and_specials(session, rows, cols, rng):
     x[4, cols - 1] = np.inf
     x[5] = np.finfo(np.float32).min
     check(A.softmax(upload(session, x, "f32"), -1).storage(), softmax_f64(x.astype(np.float64)), "f32")
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_index_select_of_many_rows(session, dtype, rng):
+    """Rows shorter and longer than a workgroup, many of them: pieces of 16, 4
+    and 2 bytes, workgroups that begin inside a row and end in another."""
+    for cols in (1, 2, 3, 7, 20, 255, 256, 257, 511, 1020, 1024, 1028, 2056):
+        x = storage(rng.standard_normal((301, cols)), dtype)
+        index = rng.integers(-3, 305, 777)
+        want = np.where(((index >= 0) & (index < 301))[:, None], x[np.clip(index, 0, 300)], 0)
+        got = A.index_select(upload(session, x, dtype), 0, session.tensor(index, "i64")).storage()
+        np.testing.assert_array_equal(got, want)
