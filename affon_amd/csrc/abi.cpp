@@ -499,7 +499,7 @@ int affon_rocm_kernel_supports(const affon_rocm_qmm_desc* desc, const char* kern
   } kGuards[] = {
       {"generic", affon::generic_supports}, {"gemv", affon::gemv_supports},     {"gemv1", affon::gemv1_supports},
       {"gemv_mfma", affon::gemv_mfma_supports}, {"mfma", affon::mfma_supports}, {"gemm_re", affon::re_gemm_supports},
-      {"gemm_pair", affon::pair_supports},  {"gemm_re32", affon::re32_supports},
+      {"gemm_pair", affon::pair_supports},  {"gemm_re32", affon::re32_supports}, {"xgemm", affon::gemv_runs_xgemm},
   };
   for (const auto& g : kGuards) {
     if (std::strcmp(g.name, kernel) == 0) {

@@ -315,28 +315,57 @@ hipError_t gemv_group_launch(const QmmProblem* group, int count, const Launch& l
 }
 
 namespace {
-// This file's kernel passes over the weights once per four rows. Where its
-// decode is cheap (8-bit codes; 2-bit codes a word at a time) and the
-// matrix-core kernel would have to split K to fill the GPU, which costs a
-// second launch, few passes over few columns are ahead. In us a call, this
-// kernel first, f32 at 8 bits and K = 4096: 2 x 4096 11.4 and 12.6, 8 x 1024
-// 8.7 and 11.2, 16 x 1024 11.3 and 11.8, 8 x 4096 20.5 and 13.4; 2-bit groups
-// of 32 2 x 4096 x 4160 11.8 and 16.1, 15 x 423 x 2624 11.3 and 14.7; from 128
-// column tiles on it is behind (14336 columns: 30.2 and 20.9). A long K leaves
-// few columns' waves too much each: K = 14336 4 x 256 15.9 and 12.4, 4 x 1024
-// 16.4 and 14.6, but 2 x 4096 21.6 and 24.5. With bf16 activations 4-bit codes
-// are a little ahead too: 2 x 1024 x 4128 9.8 and 11.0, 8 x 1024 10.5 and 11.4
-// (K = 1376, where the other needs no ranges: 9.5 and 7.9; 16 x 1024 19.2 and
-// 11.7).
+// This file's kernel passes over the weights once per four rows, a wave to
+// eight columns of a pass. It is ahead of the matrix-core kernels while its
+// waves do not fill the GPU and those have to split K (a second launch), where
+// its decode is cheap (8-bit codes; 2-bit codes a word at a time). us a call,
+// this kernel first, parameters of the activations' type:
+//
+// One row, whatever the M = 1 kernel declines it for: no product of 16 rows is
+// ahead (groups of 96, f32, 4 bits, 14336 x 14400 35 and 84, 1024 x 4032 6 and
+// 11).
+// Up to four rows, f32: at 8 bits 4 x 4096 x 4096 12.2 and 11.5, 2 of them 11.4
+// and 12.6, 4 x 14336 x 4096 31 and 22; 4 x 1024 x 14336 16.5 and 13.4; at 4
+// bits 2 x 2048 x 4096 10.2 and 10.8, 3 x 643 x 5312 10.9 and 12.8. Groups of an odd number of 32s cost the
+// other kernel a parameter pair per 32 values, so that a long K stays here: 4 x
+// 14336 x 14400 at 8 bits 76 and 104, at 2 bits 68 and 76.
+// More rows: 8 x 1024 x 4096 at 8 bits f32 8.6 and 10.7, bf16 at groups of 32
+// 8.4 and 10.6, 8 x 4096 x 4096 f32 20 and 12; at 2 bits and groups of 32 f32 16
+// x 1024 x 1344 8.8 and 12.5, 2048 columns 16.3 and 12.3; at 4 bits bf16 8 x
+// 1024 x 4096 10.2 and 9.9, 16 rows 18.5 and 9.8.
+// Past 16 rows the other kernel takes 32 at a time and is slower for few
+// columns, past 32 its tiles of 64: f32 at 4 bits and groups of 32 32 x 256 x
+// 1344 9.8 and 16.9, 1024 columns 33 and 17; 64 x 64 x 1344 9.7 and 13.5, 256
+// columns 18 and 13. Of 1245 shapes drawn over 1..181 rows, 32..19000
+// columns and K = 256..15000 a third run here; of the others the other kernel
+// is behind by over a tenth for two, by 17 % at most.
 bool few_passes_are_ahead(const QmmProblem& p) {
+  if (p.M == 1) return true;
   const int64_t columns = (p.M + 3) / 4 * p.N;  // over all passes
-  if (p.bits == 4) return p.x_dtype == AFFON_ROCM_BF16 && columns <= 2048 && p.K > 2048 && p.K <= 8192;
-  const bool two_bit_words = p.bits == 2 && p.group % 64 != 0;
-  if (p.bits == 2 && !two_bit_words) return false;
-  if (p.M <= 4) return p.N <= 8192 && (p.N > 2048 || p.K <= 8192 || two_bit_words);
-  return columns <= 4096 && p.K <= 8192;
+  const bool f32 = p.x_dtype == AFFON_ROCM_F32, odd = p.group % 64 != 0;
+  if (p.bits == 4) {
+    if (p.M > 32) return columns <= 1536 && p.K >= 512 && !(f32 && p.K > 8192);
+    if (!f32) return columns <= 2048 && p.K > 2048 && p.K <= 8192;
+    if (p.M <= 4) return p.N <= 2048 && (p.N > 1024 || p.M < 4) && p.K > 2048 && p.K < 8192;
+    return p.M > 16 && columns <= 2048 && p.K >= 1024 && p.K < 8192;
+  }
+  if (p.bits == 2 && !odd) return false;  // four words at a time
+  if (p.M <= 4) {
+    if (f32 && odd && (p.K > 8192 ? p.N > 1024 : p.bits == 8 && p.K >= 4096)) return true;
+    return p.N <= 8192 && (p.N > 2048 || p.K <= 8192 || p.bits == 2);
+  }
+  if (p.M > 32) return columns <= (p.K > 8192 ? 2304 : 4096);
+  if (p.bits == 2 && f32 && p.M > 16) {
+    if (p.K > 12288) return columns <= 2048;
+    if (p.K >= 1024 && p.K <= 2048) return columns <= 8192;
+  }
+  return columns <= 4096 && p.K <= (odd && f32 && (p.bits == 2 || p.M > 16) ? 12288 : 8192);
 }
 }  // namespace
+
+bool gemv_runs_xgemm(const QmmProblem& p) {
+  return !gemv1_supports(p) && !few_passes_are_ahead(p) && xgemm_supports(p);
+}
 
 hipError_t gemv_launch(const QmmProblem& p, const Launch& l) {
   hipStream_t stream = l.stream;
@@ -348,7 +377,7 @@ hipError_t gemv_launch(const QmmProblem& p, const Launch& l) {
       default: return gemv1_launch_b8(p, stream);
     }
   }
-  if (!few_passes_are_ahead(p) && xgemm_supports(p)) return xgemm_launch(p, l);
+  if (gemv_runs_xgemm(p)) return xgemm_launch(p, l);
   switch (p.bits) {
     case 2: return launch_bits<2>(p, stream);
     case 4: return launch_bits<4>(p, stream);

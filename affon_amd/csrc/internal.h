@@ -50,9 +50,9 @@ constexpr int kMaxGroup = 4;
 bool gemv_group_supports(const QmmProblem* group, int count);
 hipError_t gemv_group_launch(const QmmProblem* group, int count, const Launch& l);
 
-// The general matrix-core kernels (xgemm.h) that gemv_launch runs where the
-// M = 1 kernel does not take the problem.
+// The general matrix-core kernels (xgemm.h), and whether gemv_launch runs them.
 bool xgemm_supports(const QmmProblem& p);
+bool gemv_runs_xgemm(const QmmProblem& p);
 hipError_t xgemm_launch(const QmmProblem& p, const Launch& l);
 
 bool gemv_mfma_supports(const QmmProblem& p);

@@ -181,7 +181,8 @@ int affon_rocm_empty_launch(affon_rocm_session* session, uint32_t blocks, uint32
  * affon_rocm_quantized_matmul, then writes to *supported whether the guard of
  * one physical kernel behind the candidates accepts the problem (1) or not
  * (0). Kernel names: "generic", "gemv" (the gemv candidate), "gemv1" (its
- * M = 1 kernel), "gemv_mfma", "mfma", "gemm_re" (the group-scaling
+ * M = 1 kernel), "xgemm" (its matrix-core kernels: 1 where it also prefers
+ * them to the VALU kernel), "gemv_mfma", "mfma", "gemm_re" (the group-scaling
  * reassociated prefill GEMM), "gemm_re32" (the reassociated prefill GEMM for
  * groups of 32), "gemm_pair" (the 4-bit prefill GEMM); another name is
  * AFFON_ROCM_INVALID_SHAPE. Enqueues nothing. */

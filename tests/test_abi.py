@@ -264,3 +264,28 @@ def test_group32_prefill_selection():
     assert select(d) == (0, "rocm_quantized_matmul.mfma")
     d = make_desc(M=512, K=4096, N=1024, group=32, policy=_native.BACKEND_EQUIVALENT)
     assert select(d) == (0, "rocm_quantized_matmul.gemv_mfma")
+
+
+@pytest.mark.parametrize("runs,shape,bits,group,x", [
+    # One row never: what the M = 1 kernel declines runs on the VALU kernel.
+    (0, (1, 4096, 4032), 4, 96, "f32"), (0, (1, 14336, 14400), 8, 96, "bf16"), (0, (1, 14336, 4032), 2, 96, "f32"),
+    # Few columns over all passes, on both sides of the lines.
+    (0, (4, 8192, 4096), 8, 64, "f32"), (1, (4, 8193, 4096), 8, 64, "f32"), (0, (8, 2048, 8192), 8, 64, "f32"),
+    (1, (8, 2049, 8192), 8, 64, "f32"), (1, (8, 2048, 8256), 8, 64, "f32"), (0, (4, 14336, 14400), 8, 96, "f32"),
+    (1, (4, 14336, 14400), 8, 96, "bf16"), (1, (4, 14336, 1344), 8, 96, "f32"), (0, (2, 14336, 14400), 2, 96, "f32"),
+    (1, (8, 4096, 4096), 2, 64, "f32"), (1, (2, 64, 4096), 2, 64, "f32"), (0, (24, 1024, 1344), 2, 32, "f32"),
+    (1, (24, 1024, 512), 2, 32, "f32"), (0, (2, 2048, 4096), 4, 64, "f32"), (1, (4, 1024, 4096), 4, 64, "f32"),
+    (0, (3, 1024, 4096), 4, 64, "f32"), (1, (3, 2049, 4096), 4, 64, "f32"), (0, (9, 641, 11616), 2, 96, "f32"),
+    (1, (8, 1024, 4096), 4, 64, "f32"), (0, (32, 256, 4096), 4, 64, "f32"), (1, (32, 257, 4096), 4, 64, "f32"),
+    (0, (64, 64, 512), 4, 32, "bf16"), (0, (64, 96, 512), 4, 32, "bf16"), (1, (64, 97, 512), 4, 32, "bf16"), (0, (64, 256, 4096), 8, 32, "bf16"),
+    (1, (64, 257, 4096), 8, 32, "bf16"), (1, (2048, 4096, 4160), 4, 64, "bf16"),
+    # What the matrix-core kernels do not take at all.
+    (0, (64, 4096, 4096), 4, 16, "f32"), (0, (64, 4096, 4080), 4, 48, "f32"),
+])
+def test_general_batch_kernel_selection(runs, shape, bits, group, x):
+    """Which batches of the gemv candidate the matrix-core kernels run."""
+    M, N, K = shape
+    dtype = {"f32": _native.F32, "bf16": _native.BF16}[x]
+    d = make_desc(M=M, K=K, N=N, bits=bits, group=group, x_dtype=dtype, p_dtype=dtype)
+    assert kernel_supports(d, "gemv") == 1
+    assert kernel_supports(d, "xgemm") == runs
