@@ -377,7 +377,8 @@ hipError_t gemv_launch(const QmmProblem& p, const Launch& l) {
       default: return gemv1_launch_b8(p, stream);
     }
   }
-  if (gemv_runs_xgemm(p)) return xgemm_launch(p, l);
+  hipError_t status;
+  if (gemv_runs_xgemm(p) && xgemm_launch(p, l, &status)) return status;
   switch (p.bits) {
     case 2: return launch_bits<2>(p, stream);
     case 4: return launch_bits<4>(p, stream);

@@ -53,7 +53,10 @@ hipError_t gemv_group_launch(const QmmProblem* group, int count, const Launch& l
 // The general matrix-core kernels (xgemm.h), and whether gemv_launch runs them.
 bool xgemm_supports(const QmmProblem& p);
 bool gemv_runs_xgemm(const QmmProblem& p);
-hipError_t xgemm_launch(const QmmProblem& p, const Launch& l);
+// Enqueues them and returns true (*status: the launch status), or returns
+// false with nothing enqueued where the scratch memory for several K ranges
+// cannot be had now and the VALU kernel is ahead of a single one.
+bool xgemm_launch(const QmmProblem& p, const Launch& l, hipError_t* status);
 
 bool gemv_mfma_supports(const QmmProblem& p);
 hipError_t gemv_mfma_launch(const QmmProblem& p, const Launch& l);

@@ -27,6 +27,19 @@ int most_splits(const QmmProblem& p, int64_t units, int least) {
   return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(s, kMaxSplits)));
 }
 
+// Whether the VALU kernel (gemv.hip) is ahead of one K range here. A range's
+// time is that of its steps one after another, the VALU kernel's grows with the
+// columns of all its passes. f32, us, VALU kernel first: 8 x 1024 x 14336 at 4
+// bits 19 and 52, 4096 columns 72 and 53; 8 x 4096 x 4096 at 8 bits 20 and 18;
+// 64-row tiles take longer, 33 x 256 x 4096 at 4 bits 19 and 70, 2048 columns
+// 81 and 71; 64 x 1024 x 4096 at 8 bits 33 and 77, 4096 columns 114 and 77.
+bool one_range_is_behind(const QmmProblem& p) {
+  const int64_t columns = (p.M + 3) / 4 * p.N;
+  if (p.M <= 32) return p.K >= 2048 && columns <= p.K;
+  const int64_t per_k = p.bits == 4 ? 4 : p.bits == 2 && p.group % 64 == 0 ? 2 : 8;
+  return p.K >= 1024 && columns <= per_k * p.K;
+}
+
 }  // namespace
 }  // namespace xgemm
 
@@ -51,7 +64,7 @@ bool xgemm_supports(const QmmProblem& p) {
   return xgemm::ceil_div(p.M, 64) * xgemm::ceil_div(p.N, 64) <= (int64_t(1) << 27);
 }
 
-hipError_t xgemm_launch(const QmmProblem& p, const Launch& l) {
+bool xgemm_launch(const QmmProblem& p, const Launch& l, hipError_t* status) {
   using namespace xgemm;
   Args args;
   TileArgs& a = args.t;
@@ -121,18 +134,23 @@ hipError_t xgemm_launch(const QmmProblem& p, const Launch& l) {
     splits = static_cast<int>(std::min<int64_t>(most, ceil_div(want, ceil_div(p.M, bm) * ceil_div(p.N, bn))));
   }
   if (splits > 1) {
-    // Without scratch (a captured stream whose workspace cannot grow): one range.
+    // Without scratch (a captured stream whose workspace cannot grow): one
+    // range, or the VALU kernel where that fills the GPU better.
     a.partial = static_cast<float*>(l.can_split() ? l.scratch(static_cast<size_t>(splits) * p.M * p.N * 4) : nullptr);
-    if (a.partial == nullptr) splits = 1;
+    if (a.partial == nullptr) {
+      if (one_range_is_behind(p)) return false;
+      splits = 1;
+    }
   }
   a.splits = splits;
   args.unit = static_cast<int>(units / (parts * splits));
   args.extra = static_cast<int>(units % (parts * splits));
   switch (p.bits) {
-    case 2: return launch_b2(args, shape, g32, p.x_dtype, p.p_dtype, l.stream);
-    case 4: return launch_b4(args, shape, g32, p.x_dtype, p.p_dtype, l.stream);
-    default: return launch_b8(args, shape, g32, p.x_dtype, p.p_dtype, l.stream);
+    case 2: *status = launch_b2(args, shape, g32, p.x_dtype, p.p_dtype, l.stream); break;
+    case 4: *status = launch_b4(args, shape, g32, p.x_dtype, p.p_dtype, l.stream); break;
+    default: *status = launch_b8(args, shape, g32, p.x_dtype, p.p_dtype, l.stream); break;
   }
+  return true;
 }
 
 }  // namespace affon

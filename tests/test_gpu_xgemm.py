@@ -33,6 +33,13 @@ def upload_all(session, x, q, s, b, bits, x_dtype, p_dtype):
             session.from_bytes(s, A.TensorSpec(p_dtype, s.shape)), session.from_bytes(b, A.TensorSpec(p_dtype, b.shape)))
 
 
+def runs_matrix_cores(desc):
+    """Whether the gemv candidate runs the matrix-core kernels for a descriptor."""
+    runs = ctypes.c_int(-1)
+    _native.check(_native.load().affon_rocm_kernel_supports(ctypes.byref(desc), b"xgemm", ctypes.byref(runs)))
+    return runs.value == 1
+
+
 def expected_and_bound(x, q, s, b, group):
     """The product in f64, and what f32 sums of its terms may be off by: a
     term is rounded in its product with s or b and once per addition above
@@ -234,3 +241,37 @@ def test_large_bf16_activations(session, bits, M, N, K):
         assert (np.isnan(got) | (got == exact))[infinite].all()
     assert (got == exact)[infinite & (b * q > 0)].all()  # both terms of one sign
     assert np.isnan(got[np.isnan(picked)]).all()
+
+
+@pytest.mark.parametrize("M,N,bits", [(8, 1030, 4), (24, 1030, 4), (40, 256, 4), (40, 2200, 4), (130, 1500, 8)])
+def test_capture_without_scratch_on_both_sides(M, N, bits, rng):
+    """Captured on a session whose workspace is still empty: one K range, or
+    the VALU kernel where that is ahead of it (few columns for K); eager calls
+    then take several ranges. Every replay gives the same bits, within the bound."""
+    from affon_amd import ops
+    K, group = 4160, 64
+    x, q, s, b = operands(rng, M, N, K, bits, group, "f32", "f32")
+    hip = HipRuntime()
+    with A.Session("rocm") as session:
+        t = upload_all(session, x, q, s, b, bits, "f32", "f32")
+        out = session.tensor(np.full((M, N), np.nan, np.float32))
+        desc = ops._descriptor(*t, bits, group, out, "auto", "backend_equivalent")
+        assert runs_matrix_cores(desc)
+        lib = _native.load()
+
+        def enqueue():
+            assert lib.affon_rocm_quantized_matmul(session._handle, ctypes.byref(desc)) == 0, _native.last_error()
+
+        graph = hip.capture(session.stream, enqueue)
+        try:
+            want, bound = expected_and_bound(x, q, s, b, group)
+            hip.replay(session.stream, graph)
+            first = out.numpy()
+            assert (np.abs(first - want) <= bound).all()
+            for _ in range(2):
+                enqueue()
+                assert (np.abs(out.numpy() - want) <= bound).all()
+                hip.replay(session.stream, graph)
+                np.testing.assert_array_equal(out.numpy(), first)
+        finally:
+            hip.destroy(graph)
