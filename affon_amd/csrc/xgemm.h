@@ -8,7 +8,8 @@
 // bf16 MFMA operands and an f32 activation x enters as three bf16 planes,
 //   x = x1 + x2 + x3,  x1 = top 16 bits of x, x2 = top 16 bits of x - x1,
 // whose 8 + 8 + 8 significant bits hold all 24 of x (truncation, so that no
-// finite x overflows); bf16 activations are one plane. Every product is
+// finite x overflows; below 2^-110 what of x lies above 2^-133, the smallest
+// bf16 value); bf16 activations are one plane. Every product is
 // exact in f32, and each run of 64 k (32 where groups are not multiples of
 // 64) adds s * sum(x*q) + b * sum(x) in f32, as the VALU decode kernel does
 // per 16 bytes of codes: the run's term is formed first and added

@@ -39,10 +39,9 @@ def test_kept_memory_is_bounded_and_given_back():
     assert hip.free_bytes() >= before - 64 * MIB
 
 
-def test_memory_comes_back_only_when_idle(session, rng):
-    """Results whose tensors die while later work still runs keep their
-    values as long as they are held: a loop of products, each result dropped
-    two rounds later, against the first round's."""
+def test_held_results_keep_their_values(session, rng):
+    """A loop of products whose results are dropped two rounds later, so that
+    their memory goes round: those still held keep their values."""
     x = session.tensor(rng.standard_normal((64, 4096)).astype(np.float32))
     w = A.quantize(session.tensor(rng.standard_normal((4096, 4096)).astype(np.float32)), bits=4, group_size=64,
                    param_dtype="f32")

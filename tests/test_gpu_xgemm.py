@@ -7,16 +7,20 @@ import numpy as np
 import pytest
 
 import affon_amd as A
-from affon_amd import _native
+from affon_amd import _native, ops
 from tests.helpers import HipRuntime, pack_codes, storage, widened
 
 pytestmark = pytest.mark.gpu
 
 # Rows around the kernels' tiles of 16, 32, 64 and 128; columns around their 64, 128 and 256.
 SHAPES = [(2, 65), (5, 1), (16, 64), (17, 63), (32, 130), (33, 127), (64, 129), (65, 300), (129, 257)]
+# The same rows with columns enough that the matrix-core kernels, and not the VALU kernel, run them at every
+# width of codes.
+WIDE = [(2, 8200), (5, 2100), (16, 1090), (17, 1650), (32, 1030), (33, 460), (64, 300), (65, 301), (129, 257)]
 # (K, group): half a step at the end, one unit and less, odd blocks per group,
-# more groups than one parameter window, K ranges over workgroups.
-DEPTHS = [(64, 32), (160, 32), (96, 96), (576, 192), (1376, 32), (1344, 64), (2560, 128), (4160, 64)]
+# more groups than one parameter window, K ranges over workgroups; at 2 bits 96, 160, 1376 and 2592 end in
+# half of a lane's 64 codes.
+DEPTHS = [(64, 32), (160, 32), (96, 96), (576, 192), (1376, 32), (1344, 64), (2560, 128), (2592, 96), (4160, 64)]
 
 
 def operands(rng, M, N, K, bits, group, x_dtype, p_dtype):
@@ -56,8 +60,6 @@ def expected_and_bound(x, q, s, b, group):
 def test_edges_against_f64(session, bits, x_dtype, p_dtype, rng):
     for i, (K, group) in enumerate(DEPTHS):
         for M, N in SHAPES[i % 2::2] if K > 600 else SHAPES:
-            if K * bits % 128:
-                continue
             x, q, s, b = operands(rng, M, N, K, bits, group, x_dtype, p_dtype)
             t = upload_all(session, x, q, s, b, bits, x_dtype, p_dtype)
             out = session.tensor(np.full((M, N), np.nan, np.float32))
@@ -66,6 +68,27 @@ def test_edges_against_f64(session, bits, x_dtype, p_dtype, rng):
             err = np.abs(out.numpy() - want)
             assert (err <= bound).all(), (M, N, K, group, float((err / bound).max()))
             # Far below the bound in norm: no plane, block or part is missing.
+            assert np.linalg.norm(err) <= 2e-6 * np.linalg.norm(want), (M, N, K, group)
+
+
+@pytest.mark.parametrize("x_dtype,p_dtype", [("f32", "f32"), ("f32", "bf16"), ("bf16", "bf16"), ("bf16", "f32")])
+@pytest.mark.parametrize("bits", [2, 4, 8])
+def test_edges_of_the_matrix_core_kernels(session, bits, x_dtype, p_dtype, rng):
+    """As above, with columns enough that the matrix-core kernels run it all:
+    each tile, row count and end of K, every third pair of them."""
+    for i, (K, group) in enumerate(DEPTHS):
+        if x_dtype == "bf16" and bits == 4 and group % 64 == 0 and K % 256 == 0:
+            continue  # the direct-transfer kernels'
+        for M, N in [WIDE[0]] * (K < 200) + WIDE[1 + i % 3::3]:
+            x, q, s, b = operands(rng, M, N, K, bits, group, x_dtype, p_dtype)
+            t = upload_all(session, x, q, s, b, bits, x_dtype, p_dtype)
+            out = session.tensor(np.full((M, N), np.nan, np.float32))
+            desc = ops._descriptor(*t, bits, group, out, "gemv", "backend_equivalent")
+            assert runs_matrix_cores(desc), (M, N, K, group)
+            A.quantized_matmul_into(out, *t, bits=bits, group_size=group, implementation="gemv")
+            want, bound = expected_and_bound(x, q, s, b, group)
+            err = np.abs(out.numpy() - want)
+            assert (err <= bound).all(), (M, N, K, group, float((err / bound).max()))
             assert np.linalg.norm(err) <= 2e-6 * np.linalg.norm(want), (M, N, K, group)
 
 
@@ -94,6 +117,24 @@ def test_extreme_activations(session, M):
     np.testing.assert_array_equal(out.numpy()[rows], np.broadcast_to(picked[rows, None], (rows.sum(), N)))
 
 
+@pytest.mark.parametrize("M", [3, 40, 200])
+def test_smallest_activations(session, M):
+    """One nonzero f32 activation per row: its planes hold what of it lies above
+    2^-133, the smallest bf16 value, so that all bits are there from 2^-110 on;
+    below, the error stays under 2^-133."""
+    N, K, group = 70, 320, 64
+    picked = np.array([2.0 ** -109 * (2 - 2.0 ** -23), -(2.0 ** -118) * (2 - 2.0 ** -23), 2.0 ** -126, 2.0 ** -130, 2.0 ** -149],
+                      np.float32)[np.arange(M) % 5]
+    x = np.zeros((M, K), np.float32)
+    x[np.arange(M), np.arange(M) * 7 % K] = picked
+    q, s, b = np.ones((N, K), np.int64), np.full((N, K // group), 2.0 ** 30, np.float32), np.zeros((N, K // group), np.float32)
+    t = upload_all(session, x, q, s, b, 4, "f32", "f32")
+    out = session.empty("f32", (M, N))
+    A.quantized_matmul_into(out, *t, bits=4, group_size=group, implementation="gemv")
+    err = np.abs(out.numpy() * 2.0 ** -30 - picked[:, None].astype(np.float64))
+    assert (err < 2.0 ** -133).all() and (err[np.abs(picked) >= 2.0 ** -110] == 0).all()
+
+
 @pytest.mark.parametrize("M", [6, 24, 100, 300])
 def test_epilogues_and_repeats(session, M, rng):
     """Output bias and SiLU-gated product through the K ranges' reduction and
@@ -120,14 +161,14 @@ def test_epilogues_and_repeats(session, M, rng):
 def test_capture_without_scratch(M, rng):
     """Captured on a session whose workspace is still empty, the product runs
     in one K range; replays give the same bits each time, within the bound."""
-    from affon_amd import ops
-    N, K, group = 256, 4160, 64
+    N, K, group = {8: 4400, 128: 1056}[M], 4160, 64
     x, q, s, b = operands(rng, M, N, K, 8, group, "f32", "bf16")
     hip = HipRuntime()
     with A.Session("rocm") as session:
         t = upload_all(session, x, q, s, b, 8, "f32", "bf16")
         out = session.empty("f32", (M, N))
         desc = ops._descriptor(*t, 8, group, out, "auto", "backend_equivalent")
+        assert runs_matrix_cores(desc)
         lib = _native.load()
 
         def enqueue():
@@ -158,7 +199,7 @@ def test_bf16_products_start_from_their_sums(session, bits, M):
     """bf16 activations: rows of one value, whose products and sums are all
     exact, so that nothing of the start -2^(bits-1) * sum(x) may remain; an
     infinite row stays infinite with positive scales and biases."""
-    N, K, group = 70, 320, 32
+    N, K, group = 70 if bits == 4 else 8200, 320, 32
     x = np.zeros((M, K), np.float32)
     picked = np.array([1.5, -2.0 ** 60, np.inf, -np.inf, np.nan, 2.0 ** -100], np.float32)[np.arange(M) % 6]
     x[np.arange(M), np.arange(M) * 7 % K] = picked
@@ -166,19 +207,21 @@ def test_bf16_products_start_from_their_sums(session, bits, M):
     s, b = np.full((N, K // group), 2.0 ** -10, np.float32), np.full((N, K // group), 0.25, np.float32)
     t = upload_all(session, storage(x, "bf16"), q, s, b, bits, "bf16", "f32")
     out = session.empty("f32", (M, N))
+    assert runs_matrix_cores(ops._descriptor(*t, bits, group, out, "gemv", "backend_equivalent"))
     A.quantized_matmul_into(out, *t, bits=bits, group_size=group, implementation="gemv")
     want = picked * np.float32(q[0, 0] * 2.0 ** -10 + 0.25)
     np.testing.assert_array_equal(out.numpy(), np.broadcast_to(want[:, None], (M, N)))
 
 
-@pytest.mark.parametrize("M,N", [(1, 1), (3, 1), (1, 3), (33, 1), (35, 3), (33, 67), (40, 64)])
+@pytest.mark.parametrize("M,N", [(2, 1), (3, 1), (2, 3), (33, 1), (35, 3), (33, 67), (40, 64)])
 def test_reductions_of_many_ranges(session, M, N, rng):
     """32 K ranges and their ordered sum, for counts of outputs below four and
     of every remainder by four."""
-    K, bits, group = 8192, 8, 64
+    K, bits, group = 16384, 4, 64
     x, q, s, b = operands(rng, M, N, K, bits, group, "f32", "f32")
     t = upload_all(session, x, q, s, b, bits, "f32", "f32")
     out = session.tensor(np.full((M, N), np.nan, np.float32))
+    assert runs_matrix_cores(ops._descriptor(*t, bits, group, out, "gemv", "backend_equivalent"))
     A.quantized_matmul_into(out, *t, bits=bits, group_size=group, implementation="gemv")
     want, bound = expected_and_bound(x, q, s, b, group)
     err = np.abs(out.numpy() - want)
@@ -230,6 +273,7 @@ def test_large_bf16_activations(session, bits, M, N, K):
     out = session.tensor(np.full((M, N), 7.0, np.float32))
     A.quantized_matmul_into(out, *t, bits=bits, group_size=group, implementation="gemv")
     got, v = out.numpy(), picked[:, None]
+    assert runs_matrix_cores(ops._descriptor(*t, bits, group, out, "gemv", "backend_equivalent"))
     with np.errstate(over="ignore", invalid="ignore"):
         qx, bx = (q * v).astype(np.float32), (b * v).astype(np.float32)
         plain = s.astype(np.float32) * qx + bx
@@ -248,7 +292,6 @@ def test_capture_without_scratch_on_both_sides(M, N, bits, rng):
     """Captured on a session whose workspace is still empty: one K range, or
     the VALU kernel where that is ahead of it (few columns for K); eager calls
     then take several ranges. Every replay gives the same bits, within the bound."""
-    from affon_amd import ops
     K, group = 4160, 64
     x, q, s, b = operands(rng, M, N, K, bits, group, "f32", "f32")
     hip = HipRuntime()
