@@ -326,9 +326,13 @@ namespace {
 // 11).
 // Up to four rows, f32: at 8 bits 4 x 4096 x 4096 12.2 and 11.5, 2 of them 11.4
 // and 12.6, 4 x 14336 x 4096 31 and 22; 4 x 1024 x 14336 16.5 and 13.4; at 4
-// bits 2 x 2048 x 4096 10.2 and 10.8, 3 x 643 x 5312 10.9 and 12.8. Groups of an odd number of 32s cost the
-// other kernel a parameter pair per 32 values, so that a long K stays here: 4 x
-// 14336 x 14400 at 8 bits 76 and 104, at 2 bits 68 and 76.
+// bits 2 x 2048 x 4096 10.2 and 10.8, 3 x 643 x 5312 10.9 and 12.8. Where K is
+// long, one pass is bound by HBM and stays ahead for many columns: 2 x 28672 x
+// 14336 at 8 bits 115 and 122, 4 rows 134 and 125, 4 x 11008 x 8192 41 and 41.
+// Groups of an odd number of 32s also cost the other kernel a parameter pair
+// per 32 values: 4 x 14336 x 14400 at groups of 96 77 and 100, 28672 columns 143
+// and 133; at groups of 32 4 x 28672 x 14336 138 and 164, at 2 bits 112 and 124;
+// bf16 2 x 26792 x 11264 103 and 120, 4 rows 120 and 121.
 // More rows: 8 x 1024 x 4096 at 8 bits f32 8.6 and 10.7, bf16 at groups of 32
 // 8.4 and 10.6, 8 x 4096 x 4096 f32 20 and 12; at 2 bits and groups of 32 f32 16
 // x 1024 x 1344 8.8 and 12.5, 2048 columns 16.3 and 12.3; at 4 bits bf16 8 x
@@ -338,7 +342,8 @@ namespace {
 // 1344 9.8 and 16.9, 1024 columns 33 and 17; 64 x 64 x 1344 9.7 and 13.5, 256
 // columns 18 and 13. Of 1245 shapes drawn over 1..181 rows, 32..19000
 // columns and K = 256..15000 a third run here; of the others the other kernel
-// is behind by over a tenth for two, by 17 % at most.
+// is behind by over a tenth for two, by 17 % at most. Of 3192 of two to five
+// rows and 4096..28672 columns the rule's times are 0.3 % over the better ones.
 bool few_passes_are_ahead(const QmmProblem& p) {
   if (p.M == 1) return true;
   const int64_t columns = (p.M + 3) / 4 * p.N;  // over all passes
@@ -351,8 +356,12 @@ bool few_passes_are_ahead(const QmmProblem& p) {
   }
   if (p.bits == 2 && !odd) return false;  // four words at a time
   if (p.M <= 4) {
-    if (f32 && odd && (p.K > 8192 ? p.N > 1024 : p.bits == 8 && p.K >= 4096)) return true;
-    return p.N <= 8192 && (p.N > 2048 || p.K <= 8192 || p.bits == 2);
+    const bool deep = p.K >= 8192;
+    if (p.bits == 8 && p.K > 8192 && p.M < 4 && p.N > 2048 && (f32 || p.group == 32)) return true;
+    if (f32 && odd && (deep ? p.N > 1024 : p.bits == 8 && p.K >= 4096))
+      return p.N <= (p.bits == 8 && p.group != 32 ? 16384 : deep || p.M < 4 ? int64_t{1} << 31 : 20480);
+    const int64_t most = deep && (f32 || p.bits == 2) ? 12288 : f32 && odd && p.K >= 4096 ? 11264 : 8192;
+    return p.N <= most && (p.N > 2048 || p.K <= 8192 || p.bits == 2);
   }
   if (p.M > 32) return columns <= (p.K > 8192 ? 2304 : 4096);
   if (p.bits == 2 && f32 && p.M > 16) {
