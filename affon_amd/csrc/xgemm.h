@@ -99,6 +99,16 @@ __device__ __forceinline__ float centred_bias(float s, float b) {
   return kCentred<XT> ? fmaf(kCentre<BITS>, s, b) : b;
 }
 
+// f32 activations at groups of 32 on 32 x 32 products: those round down, which
+// the exact products of bf16 activations do not meet, and every step's sum came
+// out low (600 x 1024 x 12800 at 2 bits: 3.4e-7 off 64 bits, a mean of 0.83 of
+// that; VALU kernel 2.3e-7). Every other step takes -x and is subtracted, so
+// that the errors cancel: 1.9e-7. Other groups, a parameter pair per 64 values,
+// stay below the VALU kernel's error without (4.3e-7 and 2.5e-7), and the sign
+// costs them 1 % (feed-forward of 512 rows).
+template <typename XT, bool G32>
+constexpr bool kAlternate = XT::bytes == 4 && G32;
+
 // Eight consecutive activations as loaded.
 template <typename XT>
 struct Raw8 {
@@ -110,6 +120,11 @@ struct Raw8 {
   __device__ __forceinline__ void clear() {
 #pragma unroll
     for (int i = 0; i < static_cast<int>(sizeof(v) / 16); ++i) v[i] = u32x4_t{0u, 0u, 0u, 0u};
+  }
+  // Signs changed (sign 0x80000000) or kept (0), f32.
+  __device__ __forceinline__ void flip(uint32_t sign) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[XT::bytes == 4 ? i / 4 : 0][i % 4] ^= sign;
   }
   // f32 values.
   __device__ __forceinline__ float at(int i) const {
@@ -645,7 +660,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void xtile_kernel(Args args) {
     xr[i].load(base + (x_off[i] - back));
     if (G32 && half && (sq & 4)) xr[i].clear();
   };
+  // f32: the second stage holds -x (see kAlternate).
   auto write_x = [&](int i, int stage) {
+    if constexpr (kAlternate<XT, G32>) xr[i].flip(stage == 0 ? 0u : 0x80000000u);
     const float part_sum = sum8(xr[i]);
     u32x4_t pl[P];
     planes8<XT>(xr[i], P == 3 && !(fabsf(part_sum) < INFINITY), pl);
@@ -832,7 +849,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void xtile_kernel(Args args) {
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) y[rt][ct][v] += term[ct][v];
+        for (int v = 0; v < 16; ++v)
+          y[rt][ct][v] = kAlternate<XT, G32> ? fmaf(stage == 0 ? 1.0f : -1.0f, term[ct][v], y[rt][ct][v])
+                                        : y[rt][ct][v] + term[ct][v];
       __builtin_amdgcn_sched_barrier(0);
       // The next step's activations, a share after each row tile.
 #pragma unroll

@@ -318,3 +318,23 @@ def test_capture_without_scratch_on_both_sides(M, N, bits, rng):
                 np.testing.assert_array_equal(out.numpy(), first)
         finally:
             hip.destroy(graph)
+
+
+@pytest.mark.parametrize("bits", [2, 4, 8])
+def test_errors_of_many_rows_have_no_sign(session, bits, rng):
+    """f32 activations at groups of 32 in tiles of 64 rows: the products round
+    down, and the steps' errors must cancel instead of adding up. Of n errors
+    without a sign the mean is about rms / sqrt(n), here with what the outputs
+    of a row and a column share; rounding down alone gives 0.8 rms."""
+    M, N, K, group = 260, 512, 8960, 32
+    x, q, _, _ = operands(rng, M, N, K, bits, group, "f32", "f32")
+    s = np.full((N, K // group), 0.02 / (1 << bits), np.float32)
+    b = np.float32(-0.5 * ((1 << bits) - 1)) * s
+    t = upload_all(session, x, q, s, b, bits, "f32", "f32")
+    out = session.empty("f32", (M, N))
+    assert runs_matrix_cores(ops._descriptor(*t, bits, group, out, "gemv", "backend_equivalent"))
+    A.quantized_matmul_into(out, *t, bits=bits, group_size=group, implementation="gemv")
+    want, _ = expected_and_bound(x, q, s, b, group)
+    err = out.numpy() - want
+    assert abs(err.mean()) <= 0.2 * np.sqrt((err ** 2).mean())
+    assert np.linalg.norm(err) <= 2.6e-7 * np.linalg.norm(want)
