@@ -216,8 +216,9 @@ bool policy_accepts(int policy, int numerical_class) {
 // GEMM for M >= 64 (when the policy admits its approximate class), the MFMA
 // decode kernels for M >= 2 with bf16 input (the reassociated class's path
 // for prefill: from 128 rows the large-tile reassociated GEMM, gemm_re.hip,
-// where it takes the shape, else row tiles of 32), the VALU decode kernel
-// otherwise, the generic kernel last.
+// where it takes the shape, else row tiles of 32), otherwise the gemv candidate
+// (one row, f32 activations, and the layouts those decline), the generic
+// kernel last.
 bool auto_prefers(const Candidate& c, const affon::QmmProblem& p) {
   switch (c.impl) {
     case AFFON_ROCM_IMPL_MFMA: return p.M >= 64;
@@ -781,7 +782,8 @@ const char* affon_rocm_quantized_matmul_capabilities(void) {
       "\"note\":\"integer codes exact in bf16, per-group scale and bias applied in f32\"},"
       "{\"id\":\"rocm_quantized_matmul.gemv\",\"version\":1,\"numerical_class\":\"reassociated\","
       "\"guard\":\"gfx950; group_size % (32/bits) == 0; unit inner strides; aligned rows\","
-      "\"note\":\"VALU decode, f32 accumulation, per-group scale and bias applied in f32\"},"
+      "\"note\":\"one row and few passes: VALU decode; other batches with groups of 32s: matrix cores, codes exact in "
+      "bf16, f32 activations in three bf16 planes; f32 accumulation, per-group scale and bias applied in f32\"},"
       "{\"id\":\"rocm_quantized_matmul.generic\",\"version\":1,\"numerical_class\":\"exact\","
       "\"guard\":\"gfx950; any strides, byte offsets and group sizes\","
       "\"note\":\"ordered f32 loop per output, separately rounded products and sums\"}"
@@ -842,8 +844,8 @@ static int check_rows(const void* x, int32_t dtype, int64_t rows, int64_t cols, 
   if (!is_float_dtype(dtype)) return fail(AFFON_ROCM_INVALID_SHAPE, "%s requires an f32 or bf16 tensor", op);
   if (rows <= 0 || cols <= 0) return fail(AFFON_ROCM_INVALID_SHAPE, "%s requires a non-empty rank-two tensor", op);
   uint64_t count = 0;
-  // One wave per row (four rows per workgroup) or one thread per element:
-  // the grid must stay within 2^31 workgroups.
+  // Workgroups of rows stride over what a grid does not hold; one thread per
+  // element (index_select of columns) must stay within 2^31 workgroups.
   if (!mul_ok(static_cast<uint64_t>(rows), static_cast<uint64_t>(cols), &count) || count > (uint64_t(1) << 40) ||
       rows > (int64_t(1) << 32))
     return fail(AFFON_ROCM_INVALID_SHAPE, "%s size overflows", op);

@@ -11,12 +11,12 @@ namespace {
 typedef f32x4_t f32x4_word_t __attribute__((aligned(4)));
 
 // Entry i (of `count`) of every K range, added in an order that depends on
-// `splits` alone: the values V that start there. Few outputs (FEW) wait for
-// their loads, so that those of eight ranges are in flight together, and their
-// ranges may be many, so that eight are added as a tree (38 x 276 x 8320, 32
-// ranges: 1.28e-7 off 64 bits one after another). Many outputs are bound by
-// HBM and read one range after another (512 x 4096, four ranges: eight in
-// flight cost 1.5 us of 76).
+// `splits` and on whether the outputs are few for the GPU (FEW, launch_reduce):
+// the values V that start there. Few outputs wait for their loads, so that
+// those of eight ranges are in flight together, and their ranges may be many,
+// so that eight are added as a tree (38 x 276 x 8320, 32 ranges: 1.28e-7 off 64
+// bits one after another). Many outputs are bound by HBM and read one range
+// after another (512 x 4096, four ranges: eight in flight cost 1.5 us of 76).
 template <bool FEW, typename V>
 __device__ __forceinline__ V sum_ranges(const float* partial, int64_t i, int64_t count, int splits) {
   auto load = [&](int r) { return __builtin_nontemporal_load(reinterpret_cast<const V*>(partial + r * count + i)); };
