@@ -1,6 +1,7 @@
 // A stand-in for the HIP runtime, for CPU tests of memory.h: memory is host
 // memory under a limit, a stream is captured when the test says so, and
-// `device_busy` says whether work of any stream still runs.
+// `device_busy` says whether work of any stream still runs, for which hipFree
+// and hipDeviceSynchronize wait. The latter ends captures on all streams.
 #pragma once
 
 #include <cstdlib>
@@ -17,8 +18,9 @@ enum hipStreamCaptureStatus { hipStreamCaptureStatusNone = 0, hipStreamCaptureSt
 namespace fake {
 inline std::map<void*, size_t> blocks;  // what hipMalloc gave and hipFree did not take
 inline size_t used = 0, limit = size_t(1) << 40;
-inline bool session_capturing = false, session_busy = false, device_busy = false, sync_fails = false;
-inline int frees_while_capturing = 0, syncs = 0;
+inline bool session_capturing = false, session_busy = false, device_busy = false, free_fails = false;
+inline bool other_capturing = false, other_capture_broken = false;  // a capture on another stream
+inline int frees_while_capturing = 0;
 }  // namespace fake
 
 inline hipError_t hipSetDevice(int) { return hipSuccess; }
@@ -33,7 +35,9 @@ inline hipError_t hipMalloc(void** out, size_t bytes) {
 inline hipError_t hipFree(void* ptr) {
   const auto it = fake::blocks.find(ptr);
   if (it == fake::blocks.end()) throw std::logic_error("free of what is not allocated");
+  if (fake::free_fails) return hipErrorStreamCaptureUnsupported;
   fake::frees_while_capturing += fake::session_capturing;
+  fake::session_busy = fake::device_busy = false;
   fake::used -= it->second;
   fake::blocks.erase(it);  // its address is never used again, so that a second free shows
   return hipSuccess;
@@ -50,8 +54,8 @@ inline hipError_t hipStreamSynchronize(hipStream_t) {
 }
 inline hipError_t hipStreamQuery(hipStream_t) { return fake::session_busy ? hipErrorNotReady : hipSuccess; }
 inline hipError_t hipDeviceSynchronize() {
-  ++fake::syncs;
-  if (fake::session_capturing || fake::sync_fails) return hipErrorStreamCaptureUnsupported;
+  fake::other_capture_broken |= fake::other_capturing;
+  if (fake::session_capturing || fake::other_capturing) return hipErrorStreamCaptureUnsupported;
   fake::session_busy = fake::device_busy = false;
   return hipSuccess;
 }

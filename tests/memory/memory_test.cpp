@@ -42,20 +42,24 @@ bool comes_back(affon::DeviceMemory& m, const std::set<void*>& ptrs, size_t byte
 
 void reuse() {
   affon::DeviceMemory m(nullptr);
-  void* a = alloc(m, 5000);
+  void* a = alloc(m, 5 * MiB);
   free(m, a);
-  CHECK(alloc(m, 5000) == a);
+  CHECK(alloc(m, 5 * MiB) == a);
+  std::set<void*> small;
+  for (int i = 0; i < 16; ++i) small.insert(alloc(m, 5000));
+  for (void* p : small) free(m, p);
+  CHECK(small.count(alloc(m, 5000)));
 }
 
 // A block freed while any stream works waits for the device to be idle.
 void other_stream() {
   affon::DeviceMemory m(nullptr);
-  void* a = alloc(m, 5000);
+  void* a = alloc(m, 5 * MiB);
   fake::session_busy = fake::device_busy = true;
   free(m, a);
-  CHECK(alloc(m, 5000) != a && fake::device_busy);  // the session works: no wait for one block
+  CHECK(alloc(m, 5 * MiB) != a && fake::device_busy);  // the session works: no wait for one block
   fake::session_busy = false;  // only another stream works now
-  CHECK(alloc(m, 5000) == a && !fake::device_busy);
+  CHECK(alloc(m, 5 * MiB) == a && !fake::device_busy);
 }
 
 // What a captured region allocates or frees stays aside until the session ends.
@@ -99,15 +103,40 @@ void no_free_in_capture() {
   alloc(m, 64 * MiB);  // from what the parked blocks gave back
 }
 
-// The device cannot be waited for (another stream is captured): kept blocks stay, within the bound.
+// The device cannot be waited for: kept blocks stay, and none is handed out.
 void no_idle_moment() {
   affon::DeviceMemory m(nullptr);
   std::set<void*> ptrs;
   for (int i = 0; i < 20; ++i) ptrs.insert(alloc(m, 100 * MiB));
-  fake::sync_fails = true;
-  for (void* p : ptrs) free(m, p);
-  CHECK(fake::used <= 1024 * MiB);
+  fake::free_fails = true;
+  hipError_t e;
+  for (void* p : ptrs) CHECK(m.free(p, &e));
   for (int i = 0; i < 20; ++i) CHECK(!ptrs.count(alloc(m, 100 * MiB)));
+  fake::free_fails = false;
+  m.release_all();
+  CHECK(fake::blocks.empty());
+}
+
+// Allocations, frees and reuse leave a capture on another stream alone.
+void other_capture() {
+  affon::DeviceMemory m(nullptr);
+  fake::other_capturing = true;
+  void* a = alloc(m, 5 * MiB);
+  free(m, a);
+  CHECK(alloc(m, 5 * MiB) == a);
+  for (int i = 0; i < 30; ++i) free(m, alloc(m, 100 * MiB + 1000000 * i));
+  CHECK(!fake::other_capture_broken);
+}
+
+// With no memory left even for a word, kept blocks still make room.
+void full() {
+  affon::DeviceMemory m(nullptr);
+  std::set<void*> ptrs;
+  for (int i = 0; i < 4; ++i) ptrs.insert(alloc(m, MiB));
+  fake::session_busy = true;
+  for (void* p : ptrs) free(m, p);
+  fake::limit = fake::used;
+  alloc(m, 3 * MiB);
 }
 
 // A size that fits only without rounding up is still given.
@@ -190,6 +219,8 @@ int main(int, char** argv) {
   else if (name == "capture_large") capture(300 * MiB);
   else if (name == "no_free_in_capture") no_free_in_capture();
   else if (name == "no_idle_moment") no_idle_moment();
+  else if (name == "other_capture") other_capture();
+  else if (name == "full") full();
   else if (name == "exact_size") exact_size();
   else if (name == "scratch_between_threads") scratch_between_threads();
   else if (name == "host_memory_fails") host_memory_fails();

@@ -185,3 +185,38 @@ def test_scratch_between_threads(session, rng):
     for t in threads:
         t.join()
     assert not errors, errors[0]
+
+
+def test_capture_beside_another_sessions_work(rng):
+    """A capture on one session's stream while another session allocates, runs
+    and drops results, on the same thread: the capture ends well, and replays
+    give the eager result."""
+    hip = HipRuntime()
+    with A.Session("rocm") as one, A.Session("rocm") as other:
+        x = one.tensor(rng.standard_normal((8, 1024)).astype(np.float32))
+        w = A.quantize(one.tensor(rng.standard_normal((512, 1024)).astype(np.float32)), bits=4, group_size=64,
+                       param_dtype="f32")
+        out = one.empty("f32", (8, 512))
+        run = lambda: A.quantized_matmul_into(out, x, *w, bits=4, group_size=64)
+        run()
+        want = out.numpy()
+        rows = other.tensor(rng.standard_normal((8, 1024)).astype(np.float32))
+
+        def enqueue():
+            run()
+            for i in range(40):
+                result = A.softmax(rows, -1)
+                if i % 10 == 9:
+                    result.numpy()
+            run()
+
+        graph = hip.capture(one.stream, enqueue)
+        try:
+            for _ in range(3):
+                _native.check(_native.load().affon_rocm_memcpy_h2d(
+                    one._handle, out.data_ptr, np.zeros_like(want).ctypes.data, want.nbytes), "clear")
+                hip.replay(one.stream, graph)
+                np.testing.assert_array_equal(out.numpy(), want)
+                A.softmax(rows, -1)
+        finally:
+            hip.destroy(graph)
