@@ -29,12 +29,8 @@ void* Workspace::get(size_t bytes) {
     (void)hipGetLastError();
     return nullptr;
   }
-  if (hipMemset(ptr_, 0, rounded) != hipSuccess) {
-    (void)hipFree(ptr_);
-    ptr_ = nullptr;
-    (void)hipGetLastError();
-    return nullptr;
-  }
+  // Not cleared: every launch writes what a later one reads, and a memset on the
+  // null stream would invalidate captures that other streams are in.
   bytes_ = rounded;
   return ptr_;
 }

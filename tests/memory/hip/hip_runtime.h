@@ -42,7 +42,10 @@ inline hipError_t hipFree(void* ptr) {
   fake::blocks.erase(it);  // its address is never used again, so that a second free shows
   return hipSuccess;
 }
-inline hipError_t hipMemset(void*, int, size_t) { return hipSuccess; }
+inline hipError_t hipMemset(void*, int, size_t) {  // on the null stream
+  fake::other_capture_broken |= fake::other_capturing;
+  return hipSuccess;
+}
 inline hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* status) {
   *status = fake::session_capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
   return hipSuccess;

@@ -128,6 +128,12 @@ void other_capture() {
   CHECK(!fake::other_capture_broken);
 }
 
+void other_capture_scratch() {
+  affon::Workspace w(0, nullptr);
+  fake::other_capturing = true;
+  CHECK(w.get(1000) != nullptr && w.get(10 * MiB) != nullptr && !fake::other_capture_broken);
+}
+
 // With no memory left even for a word, kept blocks still make room.
 void full() {
   affon::DeviceMemory m(nullptr);
@@ -220,6 +226,7 @@ int main(int, char** argv) {
   else if (name == "no_free_in_capture") no_free_in_capture();
   else if (name == "no_idle_moment") no_idle_moment();
   else if (name == "other_capture") other_capture();
+  else if (name == "other_capture_scratch") other_capture_scratch();
   else if (name == "full") full();
   else if (name == "exact_size") exact_size();
   else if (name == "scratch_between_threads") scratch_between_threads();

@@ -188,9 +188,9 @@ def test_scratch_between_threads(session, rng):
 
 
 def test_capture_beside_another_sessions_work(rng):
-    """A capture on one session's stream while another session allocates, runs
-    and drops results, on the same thread: the capture ends well, and replays
-    give the eager result."""
+    """A capture on one session's stream while another session allocates, takes
+    its first scratch memory, runs and drops results, on the same thread: the
+    capture ends well, and replays give the eager result."""
     hip = HipRuntime()
     with A.Session("rocm") as one, A.Session("rocm") as other:
         x = one.tensor(rng.standard_normal((8, 1024)).astype(np.float32))
@@ -200,7 +200,7 @@ def test_capture_beside_another_sessions_work(rng):
         run = lambda: A.quantized_matmul_into(out, x, *w, bits=4, group_size=64)
         run()
         want = out.numpy()
-        rows = other.tensor(rng.standard_normal((8, 1024)).astype(np.float32))
+        rows = other.tensor(rng.standard_normal((3, 40000)).astype(np.float32))  # takes scratch memory
 
         def enqueue():
             run()

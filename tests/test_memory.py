@@ -18,7 +18,7 @@ def driver(tmp_path_factory):
 
 
 @pytest.mark.parametrize("check", ["reuse", "other_stream", "capture", "capture_large", "no_free_in_capture",
-                                   "no_idle_moment", "other_capture", "full", "exact_size",
+                                   "no_idle_moment", "other_capture", "other_capture_scratch", "full", "exact_size",
                                    "scratch_between_threads", "host_memory_fails"])
 def test_session_memory(driver, check):
     result = subprocess.run([str(driver), check], capture_output=True, text=True, timeout=60)
