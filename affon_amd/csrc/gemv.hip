@@ -360,7 +360,10 @@ bool few_passes_are_ahead(const QmmProblem& p) {
     if (p.bits == 8 && p.K > 8192 && p.M < 4 && p.N > 2048 && (f32 || p.group == 32)) return true;
     if (f32 && odd && (deep ? p.N > 1024 : p.bits == 8 && p.K >= 4096))
       return p.N <= (p.bits == 8 && p.group != 32 ? 16384 : deep || p.M < 4 ? int64_t{1} << 31 : 20480);
-    const int64_t most = deep && (f32 || p.bits == 2) ? 12288 : f32 && odd && p.K >= 4096 ? 11264 : 8192;
+    int64_t most = 8192;
+    if (f32 && odd && p.bits == 8 && p.K >= 3328) most = 14336;  // 2 x 14336 x 4032 at groups of 96 27 and 33
+    else if (deep && (f32 || p.bits == 2)) most = 12288;
+    else if (f32 && odd && p.K >= 4096) most = 11264;
     return p.N <= most && (p.N > 2048 || p.K <= 8192 || p.bits == 2);
   }
   if (p.M > 32) return columns <= (p.K > 8192 ? 2304 : 4096);

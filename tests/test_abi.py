@@ -281,6 +281,7 @@ def test_group32_prefill_selection():
     (1, (64, 257, 4096), 8, 32, "bf16"), (1, (2048, 4096, 4160), 4, 64, "bf16"),
     (0, (2, 26792, 11264), 8, 32, "bf16"), (1, (4, 26792, 11264), 8, 32, "bf16"), (0, (3, 28672, 14336), 8, 64, "f32"),
     (1, (4, 28672, 14336), 8, 64, "f32"), (0, (4, 12288, 8192), 8, 64, "f32"), (1, (4, 12289, 8192), 8, 64, "f32"),
+    (0, (2, 14336, 4032), 8, 96, "f32"), (1, (2, 14337, 4032), 8, 96, "f32"), (1, (2, 14336, 3264), 8, 96, "f32"),
     (0, (4, 28672, 14336), 2, 32, "f32"), (0, (4, 11264, 4096), 2, 32, "f32"), (1, (4, 11265, 4096), 2, 32, "f32"),
     # What the matrix-core kernels do not take at all.
     (0, (64, 4096, 4096), 4, 16, "f32"), (0, (64, 4096, 4080), 4, 48, "f32"),
